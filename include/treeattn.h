@@ -227,8 +227,8 @@ int ta_sparse_attn_fwd(const void* q, const void* k, const void* v, int dtype,
  * dq is deterministic.  dk and dv:
  *   ws non-NULL (ta_sparse_attn_bwd_workspace_size bytes): written (every key row, zeros where no slot names
  *     it), each key's contributions added in a fixed order (queries ascending, slots ascending) -- bit for bit
- *     reproducible.  causal: every candidate position is at most its query's position (T == Tk), which lets a
- *     key skip the queries before it.
+ *     reproducible (the slots are sorted by key in ws first).  causal: every candidate position is at most its
+ *     query's position (T == Tk); accepted for callers that know it, the result is the same.
  *   ws NULL: accumulated into with float32 atomic adds, as the reference's kernel does (zero them first); the
  *     summation order then depends on scheduling (reproducible to float32 rounding).
  */
@@ -239,7 +239,8 @@ int ta_sparse_attn_bwd(const void* q, const void* k, const void* v, const void* 
                        int B, int H, int T, int Tk, int KC, int D, float scale, void* dq, float* dk, float* dv,
                        float* ws, int causal, void* stream);
 
-/* Bytes of the deterministic route's workspace of ta_sparse_attn_bwd (per-slot ds and p, float32). */
+/* Bytes of the deterministic route's workspace of ta_sparse_attn_bwd (per-slot ds and p, the slots sorted by key and
+ * the sort's counts); 8-byte aligned. */
 int64_t ta_sparse_attn_bwd_workspace_size(int B, int H, int T, int KC);
 
 /*

@@ -1,0 +1,68 @@
+"""The sorted dk / dv route of ta_sparse_attn_bwd at the sizes where its sort and its row handling can go wrong,
+against the closed form in float64.  GPU only."""
+import math
+
+import pytest
+import torch
+
+from treeattn_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda'
+
+
+def _backward64(q, k, v, cand, scale, do):
+    """out, lse, dq, dk, dv of softmax attention over the candidate rows, float64."""
+    q, k, v, do = [x.double() for x in (q, k, v, do)]
+    B, H, T, D = q.shape
+    Tk = k.shape[2]
+    ok = (cand >= 0) & (cand < Tk)
+    out, lse = torch.zeros_like(q), torch.zeros(B, H, T, dtype=torch.float64)
+    dq, dk, dv = torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v)
+    for b in range(B):
+        for h in range(H):
+            idx = torch.where(ok[b, h], cand[b, h], 0)
+            kg, vg = k[b, h][idx], v[b, h][idx]
+            s = ((q[b, h].unsqueeze(1) * kg).sum(-1) * scale).masked_fill(~ok[b, h], -math.inf)
+            p = torch.softmax(s, -1)
+            out[b, h], lse[b, h] = (p.unsqueeze(-1) * vg).sum(1), torch.logsumexp(s, -1)
+            dp = (do[b, h].unsqueeze(1) * vg).sum(-1)
+            ds = p * (dp - (p * dp).sum(-1, keepdim=True))
+            dq[b, h] = scale * (ds.unsqueeze(-1) * kg).sum(1)
+            dk[b, h].index_add_(0, idx.reshape(-1), (scale * ds.unsqueeze(-1) * q[b, h].unsqueeze(1)).reshape(-1, D))
+            dv[b, h].index_add_(0, idx.reshape(-1), (p.unsqueeze(-1) * do[b, h].unsqueeze(1)).reshape(-1, D))
+    return out, lse, dq, dk, dv
+
+
+@pytest.mark.parametrize('T,Tk,KC,D,misaligned', [
+    (1, 1, 1, 8, False),           # one slot
+    (65, 63, 9, 24, False),        # lanes past the row, keys short of a bucket, slots past the last key
+    (2600, 2600, 12, 64, False),   # a key with more entries than one LDS tile
+    (300, 300, 70, 256, False),    # a wavefront's half per row
+    (40, 140000, 11, 8, False),    # buckets of more than 64 keys
+    (3, 500, 4200, 16, False),     # a chunk of one query, a query naming a key many times
+    (130, 130, 33, 40, True),      # rows that are not 16-byte aligned
+])
+def test_sorted_backward_matches_float64(T, Tk, KC, D, misaligned):
+    print('case', T, Tk, KC, D, misaligned, flush=True)
+    B, H = 2, 2
+    g = torch.Generator().manual_seed(T + KC)
+    q, do = (torch.randn(B, H, T, D, generator=g) for _ in range(2))
+    k, v = (torch.randn(B, H, Tk, D, generator=g) for _ in range(2))
+    cand = torch.randint(-2, Tk + 2, (B, H, T, KC), generator=g)
+    cand[..., 0] = 0               # a key every query names
+    scale = 1 / math.sqrt(D)
+    qd, kd, vd, cd, dd = (x.to(DEV) for x in (q, k, v, cand, do))
+    if misaligned:
+        qd = torch.cat([qd.new_zeros(1), qd.reshape(-1)])[1:].view(B, H, T, D)
+        dd = torch.cat([dd.new_zeros(1), dd.reshape(-1)])[1:].view(B, H, T, D)
+        assert qd.data_ptr() % 16 and dd.data_ptr() % 16
+    out, lse, *want = _backward64(q, k, v, cand, scale, do)
+    out, lse = out.float().to(DEV), lse.float().to(DEV)
+    got = K.sparse_attn_bwd(qd, kd, vd, cd, scale, out, lse, dd, deterministic=True)
+    again = K.sparse_attn_bwd(qd, kd, vd, cd, scale, out, lse, dd, deterministic=True)
+    # float32 sums of n terms: an error of about sqrt(n) * 2^-24 of the terms' norm; 1e-5 of the largest value is
+    # above that for the 2600 terms of the key that every query names
+    for a, b, w in zip(got, again, want):
+        assert torch.equal(a, b)
+        assert (a.cpu().double() - w).abs().max().item() <= 1e-5 * max(1.0, w.abs().max().item())

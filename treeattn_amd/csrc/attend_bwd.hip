@@ -3,17 +3,26 @@
 // forward's log-sum-exp), Dq = do . o, dp_j = do . v_j and ds_j = p_j (dp_j - Dq):
 //   dq = scale * sum_j ds_j k_j,   dk[cand_j] += scale * ds_j q,   dv[cand_j] += p_j do.
 //
-// sparse_attn_bwd_kernel, one wavefront per query.  Phase A, one lane per candidate slot (64 slots at a time):
-// the two dot products of its key and value rows with q and do (held in LDS and read by every lane at the same
-// address), p and ds, left in LDS.  Phase B, one lane per dimension: dq accumulates the chunk's slots in slot
-// order (so dq is deterministic).  dk and dv then take one of two routes:
-//  * with a workspace (the Python binding's default while this route's scan, quadratic in T, stays bounded):
-//    every slot's ds and p are written there, and
-//    sparse_attn_dkdv_kernel -- one workgroup per block of keys of a (sequence, head) -- scans the queries in
-//    increasing order and their slots in slot order, adding each hit on its keys into LDS accumulators, then
-//    writes the keys' rows once.  The order of the additions is fixed: dk and dv are bit-reproducible.
+// bwd_query_kernel, one wavefront per query: the valid slots of a round of 64 are compacted (typically a quarter of
+// a candidate row names a key), then 64 / L slots at a time are worked on by L lanes each (L lanes of 8 dimensions
+// hold a row): the key and value rows are read once, in whole lines, the two dot products are finished inside the
+// group, and dq takes the key row that is still in registers.  dk and dv then take one of two routes:
+//  * with a workspace (the Python binding's default while its bound holds): every valid slot's ds and p are written
+//    there, the slots are sorted by key in a stable order (queries ascending, slots ascending) and
+//    bwd_keys_kernel adds each key's contributions from its own consecutive list.  The order of the additions is
+//    fixed: dk and dv are bit-reproducible.
 //  * without one, each slot's dk and dv rows receive float32 atomic adds (the reference's scheme, whose order
 //    depends on scheduling: reproducible to float32 rounding only).
+//
+// The sort is one stable most-significant-digit pass over chunks of queries (bwd_count_kernel, bwd_scan_kernel,
+// bwd_scatter_kernel) into at most 2048 buckets of 16 (or more) consecutive keys; bwd_keys_kernel lists a bucket's
+// entries key by key in LDS.  The cost is linear in the slots.  Scanning all candidate rows once per block of keys
+// instead (one wavefront per block, a serial chain over the queries, quadratic in T) took 6.2 ms of the 7.0 ms
+// forward and backward of a (2, 6, 4096, 64) float16 layer with 52 candidates a row (12 valid); this takes 0.13 ms:
+// count 8, scan 14, scatter 18 and keys 90 us.  What is left in the key kernel is latency (about 8 us per bucket, six
+// rounds of workgroups) and the bucket of the sink, which every query names: its workgroups are started first and
+// take 85 us.  8 or 32 keys per bucket, 4 or 16 wavefronts, tiles of 1024 entries: 0.19-0.25 against 0.19 ms for the
+// whole backward.  bwd_query_kernel: 45 us (85 with a lane per slot and a second pass over the key rows).
 #include "common.hpp"
 
 namespace ta {
@@ -25,169 +34,498 @@ struct BwdParams {
   const float* lse;      // (B,H,T) contiguous
   void* dq;              // (B,H,T,D) contiguous, input dtype
   float *dk, *dv;        // (B,H,Tk,D) contiguous float32: accumulated into (atomics) or written (workspace)
-  float *ws_ds, *ws_p;   // (B,H,T,KC) per-slot ds and p (the deterministic route), or null
+  float2* dsp;           // (B,H,T,KC) per-slot (ds, p), written where the slot is valid (the sorted route), or null
+  uint2* ent;            // (B,H,T*KC) sorted entries: slot index, query << kLowBits | key within its bucket
+  int32_t* cnt;          // per (b,h): [bucket][chunk] counts, then starts; one more word: the number of entries
   int B, H, T, Tk, KC, D;
   float scale;
-  int causal;            // every candidate position <= its query's position: key blocks skip earlier queries
+  int rows_al;           // q, o and do rows, dq, dk and dv are 16-byte aligned
+  int CQ, NC;            // queries per chunk, chunks
+  int wlog, NB;          // log2 of a bucket's keys, buckets
 };
 
 constexpr int kBwdMaxD = 256;
+constexpr int kLowBits = 10;          // bits of the key within its bucket
+constexpr int kMaxBuckets = 2048;
+constexpr int kChunkSlots = 4096;     // slots per chunk (at least one query)
+constexpr int kBwdWaves = 4;          // wavefronts of the query, count and scatter kernels
+constexpr int kKeyWaves = 8;
+constexpr int kTile = 2048;           // entries sorted in LDS at a time
+constexpr int kHeavy = 96;            // a key with more entries in a tile is shared by the workgroup's wavefronts
 
+// Lanes per row: the power of two of 8-dimension slices that covers D (lanes past D hold zeros).
+__host__ __device__ constexpr int bwd_lanes(int D) {
+  int l = 1;
+  while (l * 8 < D) l *= 2;
+  return l;
+}
+
+// 8 elements at p (zeros past the row); vector loads where rows are aligned
 template <typename T>
-__global__ __launch_bounds__(kWave) void sparse_attn_bwd_kernel(BwdParams p) {
-  __shared__ float s_q[kBwdMaxD], s_do[kBwdMaxD];
-  __shared__ float s_ds[kWave], s_pw[kWave];
-  __shared__ int s_row[kWave];
-  const int lane = lane_id();
-  const int t = blockIdx.x, bh = blockIdx.y;
-  const int b = bh / p.H, h = bh - b * p.H;
-  const int D = p.D;
-  const T* qr = reinterpret_cast<const T*>(p.q) + b * p.qsb + h * p.qsh + (int64_t)t * p.qst;
-  const T* orw = reinterpret_cast<const T*>(p.o) + b * p.osb + h * p.osh + (int64_t)t * p.ost;
-  const T* dr = reinterpret_cast<const T*>(p.dout) + b * p.dsb + h * p.dsh + (int64_t)t * p.dst;
-  const T* kb = reinterpret_cast<const T*>(p.k) + b * p.ksb + h * p.ksh;
-  const T* vb = reinterpret_cast<const T*>(p.v) + b * p.vsb + h * p.vsh;
-  const int32_t* cr = p.cand + ((int64_t)bh * p.T + t) * p.KC;
-  const float lse = p.lse[(int64_t)bh * p.T + t];
-
-  // q and do to LDS; Dq = do . o (lane-strided partial sums, then the wavefront's sum)
-  float dpart = 0.0f;
-  for (int d = lane; d < D; d += kWave) {
-    const float dv_ = to_f32(dr[d]);
-    s_q[d] = to_f32(qr[d]);
-    s_do[d] = dv_;
-    dpart += dv_ * to_f32(orw[d]);
-  }
+__device__ __forceinline__ void load8(const T* p, bool in, bool al, float (&x)[8]) {
+  if (!in) {
 #pragma unroll
-  for (int o2 = 32; o2 >= 1; o2 >>= 1) dpart += __shfl_xor(dpart, o2, kWave);
-  const float Dq = dpart;
-  wave_sync();
-
-  float dq[kBwdMaxD / kWave];
+    for (int i = 0; i < 8; ++i) x[i] = 0.0f;
+  } else if (al) {
+    load_row<T, 8>(p, x);
+  } else {
 #pragma unroll
-  for (int m = 0; m < kBwdMaxD / kWave; ++m) dq[m] = 0.0f;
-  for (int c0 = 0; c0 < p.KC; c0 += kWave) {
-    // phase A: slot c0 + lane
-    const int c = c0 + lane;
-    const int j = c < p.KC ? cr[c] : -1;
-    const bool ok = j >= 0 && j < p.Tk;
-    float pw = 0.0f, ds = 0.0f;
-    if (ok) {
-      const T* kr = kb + (int64_t)j * p.kst;
-      const T* vr = vb + (int64_t)j * p.vst;
-      float s = 0.0f, dp = 0.0f;
-      for (int d0 = 0; d0 < D; d0 += 8) {
-        float kf[8], vf[8];
-        load_row<T, 8>(kr + d0, kf);
-        load_row<T, 8>(vr + d0, vf);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          s += s_q[d0 + i] * kf[i];
-          dp += s_do[d0 + i] * vf[i];
-        }
-      }
-      pw = __expf(s * p.scale - lse);
-      ds = pw * (dp - Dq);
-    }
-    s_ds[lane] = ds;
-    s_pw[lane] = pw;
-    s_row[lane] = ok ? j : -1;
-    if (p.ws_ds != nullptr && c < p.KC) {
-      const int64_t o = ((int64_t)bh * p.T + t) * p.KC + c;
-      p.ws_ds[o] = ds;
-      p.ws_p[o] = pw;
-    }
-    wave_sync();
-    // phase B: lane = dimension (and dimension + 64 m)
-    const int nc = p.KC - c0 < kWave ? p.KC - c0 : kWave;
-    for (int cc = 0; cc < nc; ++cc) {
-      const int row = s_row[cc];
-      if (row < 0) continue;
-      const float dsc = s_ds[cc], pwc = s_pw[cc];
-      const T* kr = kb + (int64_t)row * p.kst;
-      float* dkr = p.dk + ((int64_t)bh * p.Tk + row) * D;
-      float* dvr = p.dv + ((int64_t)bh * p.Tk + row) * D;
-#pragma unroll
-      for (int m = 0; m < kBwdMaxD / kWave; ++m) {
-        const int d = lane + kWave * m;
-        if (d < D) {
-          dq[m] += dsc * to_f32(kr[d]);
-          if (p.ws_ds == nullptr) {
-            atomicAdd(dkr + d, p.scale * dsc * s_q[d]);
-            atomicAdd(dvr + d, pwc * s_do[d]);
-          }
-        }
-      }
-    }
-    wave_sync();
-  }
-  T* dqr = reinterpret_cast<T*>(p.dq) + ((int64_t)bh * p.T + t) * D;
-#pragma unroll
-  for (int m = 0; m < kBwdMaxD / kWave; ++m) {
-    const int d = lane + kWave * m;
-    if (d < D) dqr[d] = from_f32<T>(p.scale * dq[m]);
+    for (int i = 0; i < 8; ++i) x[i] = to_f32(p[i]);
   }
 }
 
-// dk and dv of the keys [j0, j0 + KB) of one (sequence, head), KB = 4096 / D: one wavefront scans the queries
-// in increasing order (from j0 when causal) and, per query, its candidate slots in slot order; every slot that
-// names one of the block's keys adds scale * ds * q to that key's dk and p * do to its dv (LDS accumulators,
-// lane = dimension).  Each key's rows are written once, after the scan.
 template <typename T>
-__global__ __launch_bounds__(kWave) void sparse_attn_dkdv_kernel(BwdParams p) {
-  __shared__ float s_dk[4096], s_dv[4096];
-  const int lane = lane_id();
-  const int D = p.D, KB = 4096 / D;
-  const int j0 = blockIdx.x * KB, bh = blockIdx.y;
-  const int b = bh / p.H, h = bh - b * p.H;
-  for (int e = lane; e < KB * D; e += kWave) {
-    s_dk[e] = 0.0f;
-    s_dv[e] = 0.0f;
+__device__ __forceinline__ void store8(T* p, bool al, const float (&x)[8]) {
+  if (al) {
+    if constexpr (sizeof(T) == 4) {
+      reinterpret_cast<float4*>(p)[0] = make_float4(x[0], x[1], x[2], x[3]);
+      reinterpret_cast<float4*>(p)[1] = make_float4(x[4], x[5], x[6], x[7]);
+    } else {
+      union { T e[8]; uint4 u; } r;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) r.e[i] = from_f32<T>(x[i]);
+      *reinterpret_cast<uint4*>(p) = r.u;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] = from_f32<T>(x[i]);
   }
-  wave_sync();
-  const T* qb = reinterpret_cast<const T*>(p.q) + b * p.qsb + h * p.qsh;
-  const T* db = reinterpret_cast<const T*>(p.dout) + b * p.dsb + h * p.dsh;
-  for (int t = p.causal ? j0 : 0; t < p.T; ++t) {
-    const int32_t* cr = p.cand + ((int64_t)bh * p.T + t) * p.KC;
-    bool any = false;
-    float qv[kBwdMaxD / kWave], dov[kBwdMaxD / kWave];
-    for (int c0 = 0; c0 < p.KC; c0 += kWave) {
-      const int c = c0 + lane;
-      const int j = c < p.KC ? cr[c] : -1;
-      uint64_t hits = __ballot(j >= j0 && j < j0 + KB && j < p.Tk);
-      if (hits && !any) {   // the query's q and do rows, once
-        any = true;
+}
+
+// Sum over the lanes that hold the same slice of different slots (lane ^ multiples of L), in a fixed order.  The
+// exchanges of 8, 16 and 32 lanes are register moves: a row rotation, and the row and half swaps whose two results
+// hold a lane's own and its partner's value.
+__device__ __forceinline__ float xor16_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float xor32_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+template <int L>
+__device__ __forceinline__ float across_groups(float x) {
 #pragma unroll
-        for (int m = 0; m < kBwdMaxD / kWave; ++m) {
-          const int d = lane + kWave * m;
-          qv[m] = d < D ? to_f32(qb[(int64_t)t * p.qst + d]) : 0.0f;
-          dov[m] = d < D ? to_f32(db[(int64_t)t * p.dst + d]) : 0.0f;
-        }
+  for (int o = L; o < 8; o *= 2) x += __shfl_xor(x, o, kWave);
+  if constexpr (L <= 8) x += dpp_f<0x128>(x);   // row_ror:8
+  if constexpr (L <= 16) x = xor16_sum(x);
+  return xor32_sum(x);
+}
+
+template <typename T, int L>
+__global__ __launch_bounds__(kWave * kBwdWaves) void bwd_query_kernel(BwdParams p) {
+  constexpr int G = kWave / L;   // slots worked on together
+  __shared__ int s_row[kBwdWaves][kWave], s_slot[kBwdWaves][kWave];
+  const int lane = lane_id(), wv = wave_id();
+  const int t = blockIdx.x * kBwdWaves + wv, bh = blockIdx.y;
+  if (t >= p.T) return;   // a whole wavefront leaves; no workgroup barrier follows
+  const int b = bh / p.H, h = bh - b * p.H;
+  const int D = p.D;
+  const int g = lane / L, d0 = (lane % L) * 8;
+  const bool in = d0 < D;
+  const bool al = p.rows_al != 0;
+  const T* kb = reinterpret_cast<const T*>(p.k) + b * p.ksb + h * p.ksh + d0;
+  const T* vb = reinterpret_cast<const T*>(p.v) + b * p.vsb + h * p.vsh + d0;
+  const int64_t row = (int64_t)bh * p.T + t;
+  const int32_t* cr = p.cand + row * p.KC;
+  const float lse = p.lse[row];
+  float qf[8], df[8], of[8];
+  load8(reinterpret_cast<const T*>(p.q) + b * p.qsb + h * p.qsh + (int64_t)t * p.qst + d0, in, al, qf);
+  load8(reinterpret_cast<const T*>(p.dout) + b * p.dsb + h * p.dsh + (int64_t)t * p.dst + d0, in, al, df);
+  load8(reinterpret_cast<const T*>(p.o) + b * p.osb + h * p.osh + (int64_t)t * p.ost + d0, in, al, of);
+  float Dq = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) Dq += df[i] * of[i];
+  Dq = group_sum<L>(Dq);
+  float dq[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) dq[i] = 0.0f;
+  const uint64_t below = (1ull << lane) - 1;
+  for (int c0 = 0; c0 < p.KC; c0 += kWave) {
+    const int c = c0 + lane;
+    const int j = c < p.KC ? cr[c] : -1;
+    const bool ok = j >= 0 && j < p.Tk;
+    const uint64_t m = __ballot(ok);
+    const int n = __popcll(m);
+    if (ok) {
+      const int r = __popcll(m & below);
+      s_row[wv][r] = j;
+      s_slot[wv][r] = c;
+    }
+    wave_sync();
+    for (int i = g; i - g < n; i += G) {
+      const bool live = i < n;
+      const int jr = live ? s_row[wv][i] : 0;
+      float kf[8], vf[8];
+      load8(kb + (int64_t)jr * p.kst, in && live, true, kf);
+      load8(vb + (int64_t)jr * p.vst, in && live, true, vf);
+      float s = 0.0f, dp = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        s += qf[e] * kf[e];
+        dp += df[e] * vf[e];
       }
-      while (hits) {   // the hits in slot order
-        const int hl = __ffsll((unsigned long long)hits) - 1;
-        hits &= hits - 1;
-        const int key = __shfl(j, hl, kWave) - j0;
-        const int64_t o = ((int64_t)bh * p.T + t) * p.KC + c0 + hl;
-        const float dsv = p.ws_ds[o], pwv = p.ws_p[o];
+      s = group_sum<L>(s);
+      dp = group_sum<L>(dp);
+      const float pw = live ? __expf(s * p.scale - lse) : 0.0f;
+      const float ds = live ? pw * (dp - Dq) : 0.0f;
 #pragma unroll
-        for (int m = 0; m < kBwdMaxD / kWave; ++m) {
-          const int d = lane + kWave * m;
-          if (d < D) {
-            s_dk[key * D + d] += p.scale * dsv * qv[m];
-            s_dv[key * D + d] += pwv * dov[m];
+      for (int e = 0; e < 8; ++e) dq[e] += ds * kf[e];
+      if (live) {
+        if (p.dsp != nullptr) {
+          if (d0 == 0) p.dsp[row * p.KC + s_slot[wv][i]] = make_float2(ds, pw);
+        } else if (in) {
+          float* dkr = p.dk + ((int64_t)bh * p.Tk + jr) * D + d0;
+          float* dvr = p.dv + ((int64_t)bh * p.Tk + jr) * D + d0;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            atomicAdd(dkr + e, p.scale * ds * qf[e]);
+            atomicAdd(dvr + e, pw * df[e]);
           }
         }
       }
     }
+    wave_sync();
   }
-  wave_sync();
-  for (int e = lane; e < KB * D; e += kWave) {
-    const int key = j0 + e / D;
-    if (key < p.Tk) {
-      p.dk[((int64_t)bh * p.Tk + key) * D + e % D] = s_dk[e];
-      p.dv[((int64_t)bh * p.Tk + key) * D + e % D] = s_dv[e];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) dq[e] = p.scale * across_groups<L>(dq[e]);
+  if (g == 0 && in) store8(reinterpret_cast<T*>(p.dq) + row * D + d0, al, dq);
+}
+
+// ---------------------------------------------------------------------------------- sorting the slots by key
+// A chunk's slots are consecutive: queries [ch * CQ, ...), KC slots each.
+__device__ __forceinline__ void chunk_range(const BwdParams& p, int ch, int& s0, int& s1) {
+  const int t0 = ch * p.CQ, t1 = t0 + p.CQ < p.T ? t0 + p.CQ : p.T;
+  s0 = t0 * p.KC;
+  s1 = t1 * p.KC;
+}
+
+__global__ __launch_bounds__(kWave * kBwdWaves) void bwd_count_kernel(BwdParams p) {
+  __shared__ int s_n[kMaxBuckets];
+  const int ch = blockIdx.x, bh = blockIdx.y;
+  for (int i = threadIdx.x; i < p.NB; i += blockDim.x) s_n[i] = 0;
+  __syncthreads();
+  int s0, s1;
+  chunk_range(p, ch, s0, s1);
+  const int32_t* cr = p.cand + (int64_t)bh * p.T * p.KC;
+  for (int s = s0 + threadIdx.x; s < s1; s += blockDim.x) {
+    const int j = cr[s];
+    if (j >= 0 && j < p.Tk) atomicAdd(&s_n[j >> p.wlog], 1);
+  }
+  __syncthreads();
+  int32_t* cnt = p.cnt + (int64_t)bh * ((int64_t)p.NB * p.NC + 1);
+  for (int i = threadIdx.x; i < p.NB; i += blockDim.x) cnt[(int64_t)i * p.NC + ch] = s_n[i];
+}
+
+// Exclusive sums of one (b,h)'s counts, in place, and the number of entries after them: 8 counts per thread and step.
+__global__ __launch_bounds__(1024) void bwd_scan_kernel(BwdParams p) {
+  __shared__ int s_w[16];
+  const int n = p.NB * p.NC;
+  int32_t* cnt = p.cnt + (int64_t)blockIdx.x * ((int64_t)n + 1);
+  const int lane = lane_id(), wv = wave_id();
+  int base = 0;
+  for (int i0 = 0; i0 < n; i0 += 8192) {
+    int x[8], sum = 0;
+    const int i = i0 + (int)threadIdx.x * 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      x[e] = i + e < n ? cnt[i + e] : 0;
+      sum += x[e];
     }
+    int inc = sum;   // inclusive over the wavefront
+#pragma unroll
+    for (int o = 1; o < kWave; o *= 2) {
+      const int y = __shfl_up(inc, o, kWave);
+      if (lane >= o) inc += y;
+    }
+    if (lane == kWave - 1) s_w[wv] = inc;
+    __syncthreads();
+    int before = base, all = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      if (w < wv) before += s_w[w];
+      all += s_w[w];
+    }
+    int at = before + inc - sum;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if (i + e < n) cnt[i + e] = at;
+      at += x[e];
+    }
+    base += all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) cnt[n] = base;
+}
+
+// Lanes of the wavefront that hold the same digit (`bits` wide) as this one, among the valid ones.
+__device__ __forceinline__ uint64_t same_digit(int digit, bool ok, int bits) {
+  uint64_t m = __ballot(ok);
+  for (int b = 0; b < bits; ++b) {
+    const bool one = (digit >> b) & 1;
+    const uint64_t y = __ballot(one);
+    m &= one ? y : ~y;
+  }
+  return m;
+}
+
+// Each chunk's valid slots to their places: bucket starts from the scan, then wavefronts (a consecutive quarter of
+// the chunk each), rounds of 64 slots and lanes in order -- a stable order.
+__global__ __launch_bounds__(kWave * kBwdWaves) void bwd_scatter_kernel(BwdParams p) {
+  __shared__ int s_n[kBwdWaves][kMaxBuckets];
+  const int ch = blockIdx.x, bh = blockIdx.y;
+  const int lane = lane_id(), wv = wave_id();
+  int* mine = s_n[wv];
+  for (int i = lane; i < p.NB; i += kWave) mine[i] = 0;
+  wave_sync();
+  int s0, s1;
+  chunk_range(p, ch, s0, s1);
+  const int part = (s1 - s0 + kBwdWaves - 1) / kBwdWaves;
+  const int a0 = s0 + wv * part, a1 = a0 + part < s1 ? a0 + part : s1;
+  const int32_t* cr = p.cand + (int64_t)bh * p.T * p.KC;
+  for (int s = a0 + lane; s < a1; s += kWave) {
+    const int j = cr[s];
+    if (j >= 0 && j < p.Tk) atomicAdd(&mine[j >> p.wlog], 1);
+  }
+  __syncthreads();
+  const int32_t* cnt = p.cnt + (int64_t)bh * ((int64_t)p.NB * p.NC + 1);
+  for (int i = threadIdx.x; i < p.NB; i += blockDim.x) {
+    int at = cnt[(int64_t)i * p.NC + ch];
+#pragma unroll
+    for (int w = 0; w < kBwdWaves; ++w) {
+      const int n = s_n[w][i];
+      s_n[w][i] = at;
+      at += n;
+    }
+  }
+  __syncthreads();
+  uint2* ent = p.ent + (int64_t)bh * p.T * p.KC;
+  const int bits = 32 - __clz(p.NB - 1 | 1);
+  const uint64_t below = (1ull << lane) - 1;
+  const int low = (1 << p.wlog) - 1;
+  for (int sb = a0; sb < a1; sb += kWave) {
+    const int s = sb + lane;
+    const int j = s < a1 ? cr[s] : -1;
+    const bool ok = j >= 0 && j < p.Tk;
+    const int d = ok ? j >> p.wlog : 0;
+    const uint64_t m = same_digit(d, ok, bits);
+    int at = 0;
+    if (ok) at = mine[d] + __popcll(m & below);
+    wave_sync();
+    if (ok) {
+      ent[at] = make_uint2((uint32_t)s, (uint32_t)(s / p.KC) << kLowBits | (uint32_t)(j & low));
+      if ((m >> lane) == 1) mine[d] = at + 1;   // the last lane of the digit
+    }
+    wave_sync();
+  }
+}
+
+// ------------------------------------------------------------------------------------------------ dk and dv
+// 8 elements of a row as they lie in memory, converted when they are used (fewer registers for rows in flight)
+template <typename T>
+struct Raw8 {
+  T e[8];
+  __device__ __forceinline__ void load(const T* p, bool vec) {
+    if (vec) {
+#pragma unroll
+      for (int i = 0; i < (int)sizeof(T) / 2; ++i)
+        reinterpret_cast<uint4*>(e)[i] = reinterpret_cast<const uint4*>(p)[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) e[i] = p[i];
+    }
+  }
+};
+
+// Contributions of entries list[g], list[g + G], ... < n of one key to its dk and dv slices (this lane's group's
+// part), then their sum over the groups.  BATCH entries' rows are requested together (past the end the last entry's,
+// with weight 0), so that a list pays one round trip per BATCH * G entries.
+template <typename T, int L, bool VEC, int BATCH>
+__device__ __forceinline__ void key_part(const BwdParams& p, const T* qb, const T* db, const float2* dsp,
+                                         const uint2* s_e, const uint16_t* list, int n, int g, float (&dk)[8],
+                                         float (&dv)[8]) {
+  constexpr int G = kWave / L;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) dk[i] = dv[i] = 0.0f;
+  for (int i0 = 0; i0 < n; i0 += G * BATCH) {
+    float2 c[BATCH];
+    Raw8<T> qr[BATCH], dr[BATCH];
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u) {
+      const int i = i0 + u * G + g;
+      const uint2 e = s_e[list[i < n ? i : n - 1]];
+      const int64_t t = e.y >> kLowBits;
+      c[u] = dsp[e.x];
+      qr[u].load(qb + t * p.qst, VEC);
+      dr[u].load(db + t * p.dst, VEC);
+    }
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u) {
+      const bool live = i0 + u * G + g < n;
+      const float a = live ? p.scale * c[u].x : 0.0f, w = live ? c[u].y : 0.0f;
+#pragma unroll
+      for (int x = 0; x < 8; ++x) {
+        dk[x] += a * (live ? to_f32(qr[u].e[x]) : 0.0f);
+        dv[x] += w * (live ? to_f32(dr[u].e[x]) : 0.0f);
+      }
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    dk[x] = across_groups<L>(dk[x]);
+    dv[x] = across_groups<L>(dv[x]);
+  }
+}
+
+// dk and dv of one bucket's keys of one (sequence, head).  The bucket's entries come through LDS a tile at a time;
+// per round every wavefront takes one key, lists the tile's entries of that key (ballots over the tile, which keeps
+// their order) and adds their contributions, 64 / L entries at a time (the q and do rows in whole lines, the groups'
+// partial sums in a fixed order).  A key that many queries name (the sink) is shared by all wavefronts, their parts
+// added in order.  Each row is written by the first tile and added to by later ones.
+template <typename T, int L, bool VEC>
+__global__ __launch_bounds__(kWave * kKeyWaves, 4) void bwd_keys_kernel(BwdParams p) {
+  __shared__ uint2 s_e[kTile];
+  __shared__ uint16_t s_list[kKeyWaves][kTile];
+  __shared__ uint8_t s_heavy[1 << kLowBits];
+  __shared__ float s_part[kKeyWaves][2][L * 8];
+  const int lane = lane_id(), wv = wave_id(), tid = threadIdx.x;
+  const int bh = blockIdx.x, bk = blockIdx.y;   // first buckets first: they hold the sink, the longest list
+  const int b = bh / p.H, h = bh - b * p.H;
+  const int D = p.D;
+  const int g = lane / L, d0 = (lane % L) * 8;
+  const bool in = d0 < D;
+  const int j0 = bk << p.wlog;
+  const int W = 1 << p.wlog;
+  const int nk = p.Tk - j0 < W ? p.Tk - j0 : W;
+  const int32_t* cnt = p.cnt + (int64_t)bh * ((int64_t)p.NB * p.NC + 1);
+  const int first = cnt[(int64_t)bk * p.NC], last = cnt[(int64_t)(bk + 1) * p.NC];
+  const uint2* ent = p.ent + (int64_t)bh * p.T * p.KC;
+  const float2* dsp = p.dsp + (int64_t)bh * p.T * p.KC;
+  const int dl = in ? d0 : 0;   // lanes past the row read its first slice and write nothing
+  const T* qb = reinterpret_cast<const T*>(p.q) + b * p.qsb + h * p.qsh + dl;
+  const T* db = reinterpret_cast<const T*>(p.dout) + b * p.dsb + h * p.dsh + dl;
+  float* dkb = p.dk + ((int64_t)bh * p.Tk + j0) * D;
+  float* dvb = p.dv + ((int64_t)bh * p.Tk + j0) * D;
+  const uint64_t below = (1ull << lane) - 1;
+  constexpr uint32_t kLow = (1u << kLowBits) - 1;
+  uint16_t* list = s_list[wv];
+  // this wavefront's list of the entries i0 <= i < i1 of the tile that name `key`
+  auto find = [&](int key, int i0, int i1) {
+    int len = 0;
+#pragma unroll 4
+    for (; i0 < i1; i0 += kWave) {
+      const int i = i0 + lane;
+      const bool mine = i < i1 && (s_e[i].y & kLow) == (uint32_t)key;
+      const uint64_t m = __ballot(mine);
+      if (mine) list[len + __popcll(m & below)] = (uint16_t)i;
+      len += __popcll(m);
+    }
+    wave_sync();
+    return len;
+  };
+  float dk[8], dv[8];
+  int at = first;
+  do {
+    const bool fresh = at == first;
+    const int n = last - at < kTile ? last - at : kTile;
+    for (int i = tid; i < n; i += kWave * kKeyWaves) s_e[i] = ent[at + i];
+    __syncthreads();
+    for (int key = wv; key < W; key += kKeyWaves) {
+      const int len = key < nk ? find(key, 0, n) : 0;
+      if (lane == 0) s_heavy[key] = len > kHeavy;
+      if (key >= nk || len > kHeavy || (len == 0 && !fresh)) continue;
+      key_part<T, L, VEC, 2>(p, qb, db, dsp, s_e, list, len, g, dk, dv);
+      if (g == 0 && in) {
+        float* dkr = dkb + (int64_t)key * D + d0;
+        float* dvr = dvb + (int64_t)key * D + d0;
+        if (!fresh) {
+#pragma unroll
+          for (int x = 0; x < 8; ++x) {
+            dk[x] += dkr[x];
+            dv[x] += dvr[x];
+          }
+        }
+        store8(dkr, VEC, dk);
+        store8(dvr, VEC, dv);
+      }
+    }
+    __syncthreads();
+    for (int key = 0; key < nk; ++key) {   // the keys with many entries: a consecutive part of the tile per wavefront
+      if (!s_heavy[key]) continue;
+      const int part = (n + kKeyWaves - 1) / kKeyWaves;
+      const int i0 = wv * part, i1 = i0 + part < n ? i0 + part : n;
+      const int len = find(key, i0, i1);
+      key_part<T, L, VEC, sizeof(T) == 4 ? 4 : 8>(p, qb, db, dsp, s_e, list, len, g, dk, dv);
+      if (g == 0) {
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          s_part[wv][0][d0 + x] = dk[x];
+          s_part[wv][1][d0 + x] = dv[x];
+        }
+      }
+      __syncthreads();
+      for (int d = tid; d < 2 * D; d += kWave * kKeyWaves) {
+        const int which = d >= D, dd = which ? d - D : d;
+        float sum = 0.0f;
+#pragma unroll
+        for (int u = 0; u < kKeyWaves; ++u) sum += s_part[u][which][dd];
+        float* r = (which ? dvb : dkb) + (int64_t)key * D + dd;
+        *r = fresh ? sum : *r + sum;
+      }
+      __syncthreads();
+    }
+    at += n;
+    __syncthreads();   // the tile is rewritten
+  } while (at < last);
+}
+
+__global__ void bwd_zero_kernel(float* a, float* b, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    a[i] = b[i] = 0.0f;
+}
+
+// Chunks, buckets and workspace words (float32) of the sorted route.
+struct BwdPlan {
+  int CQ, NC, wlog, NB;
+  bool ok;   // the slot and query indices fit the entries
+};
+
+static BwdPlan bwd_plan(int T, int Tk, int KC) {
+  BwdPlan r;
+  r.CQ = KC >= kChunkSlots ? 1 : kChunkSlots / KC;
+  r.NC = (T + r.CQ - 1) / r.CQ;
+  r.wlog = 4;   // 16 keys: two per wavefront of the key kernel
+  while (((Tk - 1) >> r.wlog) + 1 > kMaxBuckets) ++r.wlog;
+  r.NB = ((Tk - 1) >> r.wlog) + 1;
+  r.ok = (int64_t)T * KC < (1ll << 31) - (1 << 16) && T <= (1 << (32 - kLowBits)) && r.wlog <= kLowBits;
+  return r;
+}
+
+template <typename T, int L>
+static void launch_bwd(const BwdParams& p, bool sorted, hipStream_t st) {
+  const dim3 block(kWave * kBwdWaves);
+  const unsigned bh = (unsigned)(p.B * p.H);
+  hipLaunchKernelGGL((bwd_query_kernel<T, L>), dim3((unsigned)((p.T + kBwdWaves - 1) / kBwdWaves), bh), block, 0, st, p);
+  if (!sorted) return;
+  hipLaunchKernelGGL(bwd_count_kernel, dim3((unsigned)p.NC, bh), block, 0, st, p);
+  hipLaunchKernelGGL(bwd_scan_kernel, dim3(bh), dim3(1024), 0, st, p);
+  hipLaunchKernelGGL(bwd_scatter_kernel, dim3((unsigned)p.NC, bh), block, 0, st, p);
+  const dim3 kgrid(bh, (unsigned)p.NB), kblock(kWave * kKeyWaves);
+  if (p.rows_al)
+    hipLaunchKernelGGL((bwd_keys_kernel<T, L, true>), kgrid, kblock, 0, st, p);
+  else
+    hipLaunchKernelGGL((bwd_keys_kernel<T, L, false>), kgrid, kblock, 0, st, p);
+}
+
+template <typename T>
+static void launch_bwd_d(const BwdParams& p, bool sorted, hipStream_t st) {
+  switch (bwd_lanes(p.D)) {
+    case 1: launch_bwd<T, 1>(p, sorted, st); break;
+    case 2: launch_bwd<T, 2>(p, sorted, st); break;
+    case 4: launch_bwd<T, 4>(p, sorted, st); break;
+    case 8: launch_bwd<T, 8>(p, sorted, st); break;
+    case 16: launch_bwd<T, 16>(p, sorted, st); break;
+    default: launch_bwd<T, 32>(p, sorted, st); break;
   }
 }
 
@@ -221,31 +559,42 @@ extern "C" int ta_sparse_attn_bwd(const void* q, const void* k, const void* v, c
     set_error("ta_sparse_attn_bwd: B * H above 65535");
     return TA_ERR_UNSUPPORTED;
   }
-  float* ws_ds = ws;
-  float* ws_p = ws != nullptr ? ws + (int64_t)B * H * T * KC : nullptr;
+  // rows of q, o, dout, dq, dk and dv are moved 8 elements at a time where all are aligned, else one by one
+  const int al = !(((uintptr_t)q | (uintptr_t)o | (uintptr_t)dout | (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) % 16 || (qsb * es) % 16 || (qsh * es) % 16 ||
+                   (qst * es) % 16 || (osb * es) % 16 || (osh * es) % 16 || (ost * es) % 16 || (dsb * es) % 16 ||
+                   (dsh * es) % 16 || (dst * es) % 16);
   BwdParams p{q, k, v, o, dout, qsb, qsh, qst, ksb, ksh, kst, vsb, vsh, vst, osb, osh, ost, dsb, dsh, dst,
-              cand, lse, dq, dk, dv, ws_ds, ws_p, B, H, T, Tk, KC, D, scale, causal};
-  const dim3 grid((unsigned)T, (unsigned)(B * H));
+              cand, lse, dq, dk, dv, nullptr, nullptr, nullptr, B, H, T, Tk, KC, D, scale, al, 0, 0, 0, 0};
   hipStream_t st = (hipStream_t)stream;
-  switch (dtype) {
-    case TA_F32: hipLaunchKernelGGL(sparse_attn_bwd_kernel<float>, grid, dim3(kWave), 0, st, p); break;
-    case TA_F16: hipLaunchKernelGGL(sparse_attn_bwd_kernel<f16_t>, grid, dim3(kWave), 0, st, p); break;
-    default: hipLaunchKernelGGL(sparse_attn_bwd_kernel<bf16_t>, grid, dim3(kWave), 0, st, p); break;
+  bool sorted = ws != nullptr && KC > 0;
+  if (sorted) {
+    const BwdPlan pl = bwd_plan(T, Tk, KC);
+    const int64_t slots = (int64_t)B * H * T * KC;
+    sorted = pl.ok;
+    p.dsp = reinterpret_cast<float2*>(ws);
+    p.ent = reinterpret_cast<uint2*>(ws + 2 * slots);
+    p.cnt = reinterpret_cast<int32_t*>(ws + 4 * slots);
+    p.CQ = pl.CQ, p.NC = pl.NC, p.wlog = pl.wlog, p.NB = pl.NB;
   }
-  int rc = check_launch("sparse_attn_bwd_kernel");
-  if (rc != TA_OK || ws == nullptr) return rc;
-  const int KB = 4096 / D;
-  const dim3 kgrid((unsigned)((Tk + KB - 1) / KB), (unsigned)(B * H));
-  switch (dtype) {
-    case TA_F32: hipLaunchKernelGGL(sparse_attn_dkdv_kernel<float>, kgrid, dim3(kWave), 0, st, p); break;
-    case TA_F16: hipLaunchKernelGGL(sparse_attn_dkdv_kernel<f16_t>, kgrid, dim3(kWave), 0, st, p); break;
-    default: hipLaunchKernelGGL(sparse_attn_dkdv_kernel<bf16_t>, kgrid, dim3(kWave), 0, st, p); break;
+  if (ws != nullptr && !sorted) {   // indices past the entries' 32 bits, or no slots: atomic adds into cleared rows
+    p.dsp = nullptr;
+    const int64_t n = (int64_t)B * H * Tk * D;
+    const int64_t wgs = (n + 255) / 256;
+    hipLaunchKernelGGL(bwd_zero_kernel, dim3((unsigned)(wgs < 4096 ? wgs : 4096)), dim3(256), 0, st, dk, dv, n);
   }
-  return check_launch("sparse_attn_dkdv_kernel");
+  switch (dtype) {
+    case TA_F32: launch_bwd_d<float>(p, sorted, st); break;
+    case TA_F16: launch_bwd_d<f16_t>(p, sorted, st); break;
+    default: launch_bwd_d<bf16_t>(p, sorted, st); break;
+  }
+  return check_launch("ta_sparse_attn_bwd");
 }
 
-// Workspace of the deterministic dk / dv route of ta_sparse_attn_bwd: per-slot ds and p, float32.
+// Workspace of the sorted dk / dv route of ta_sparse_attn_bwd: per-slot (ds, p), the sorted entries, and the counts of
+// at most kMaxBuckets buckets per chunk of queries (whatever the number of keys).
 extern "C" int64_t ta_sparse_attn_bwd_workspace_size(int B, int H, int T, int KC) {
   if (B <= 0 || H <= 0 || T <= 0 || KC <= 0) return 0;
-  return 2 * (int64_t)B * H * T * KC * (int64_t)sizeof(float);
+  const BwdPlan pl = bwd_plan(T, 1, KC);
+  const int64_t bh = (int64_t)B * H;
+  return (4 * bh * T * KC + bh * ((int64_t)kMaxBuckets * pl.NC + 1)) * (int64_t)sizeof(float);
 }

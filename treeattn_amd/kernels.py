@@ -601,14 +601,15 @@ def sparse_attn_fwd(q, k, v, cand, scale):
     return out, lse
 
 
-# The deterministic dk/dv route reads, for every block of 4096 / D keys, the candidate row of every query at or
-# after the block (causal) or of every query: (T / block) * T * KC int32 per (sequence, head), quadratic in T.
-# Above this many int32 reads in all (8 GiB, about 1.7 ms of HBM time) the default is the atomic route.
+# Where the default leaves the deterministic dk/dv route for the atomic one, as a count that grows with the square
+# of T (dkdv_scan_ints).  The deterministic route sorts the slots by key, whose time is linear in them, but holds 16
+# bytes per candidate slot while the backward runs; the line keeps that below a few GB at training lengths.
 DKDV_SCAN_LIMIT = 2 ** 31
 
 
 def dkdv_scan_ints(B, H, T, Tk, KC, D, causal):
-    """int32 reads of the deterministic dk/dv route's scan: per key block, the candidate rows it scans."""
+    """Candidate entries at or after each block of 4096 / D keys (causal; else all of them), over the blocks: what
+    DKDV_SCAN_LIMIT bounds."""
     KB = max(1, 4096 // max(D, 1))
     nblk = (Tk + KB - 1) // KB
     rows = sum(T - min(j * KB, T) for j in range(nblk)) if causal else nblk * T
@@ -617,11 +618,10 @@ def dkdv_scan_ints(B, H, T, Tk, KC, D, causal):
 
 def sparse_attn_bwd(q, k, v, cand, scale, out, lse, dout, deterministic=None, causal=False):
     """Gradients of sparse_attn_fwd: (dq in q's dtype, dk, dv in k's / v's dtype).  dk and dv are summed in
-    float32: deterministic, in a fixed order (queries, then slots, ascending) through a per-slot workspace; else
-    with atomic adds whose order depends on scheduling, as in the reference's kernel.  deterministic=None (the
-    default) takes the fixed order while its scan (dkdv_scan_ints) stays within DKDV_SCAN_LIMIT, the atomic adds
-    above it (long training contexts: the scan grows as T^2).  causal: every candidate position is at most its
-    query's position (lets the deterministic route skip earlier queries)."""
+    float32: deterministic, in a fixed order (the slots sorted by key, queries then slots ascending) through a
+    per-slot workspace; else with atomic adds whose order depends on scheduling, as in the reference's kernel.
+    deterministic=None (the default) takes the fixed order while dkdv_scan_ints stays within DKDV_SCAN_LIMIT, the
+    atomic adds above it.  causal: every candidate position is at most its query's position."""
     L.require_gpu(q, k, v, cand, out, lse, dout)
     if not (q.dtype == k.dtype == v.dtype == out.dtype):
         raise TypeError('q, k, v and out must share a dtype')

@@ -204,6 +204,21 @@ int ta_assemble_candidates(const int64_t* tree_pos, const uint8_t* leaf_ok, cons
                            int leaf, int nbk, int local, int32_t* cm, int32_t* counts, void* stream);
 
 /*
+ * The same masked candidate list from a selection's leaves (seg.py:111-119, fastseg.py:367-381): ids int32 and vld
+ * (B,H,N,wl) as a descent writes them, lhat int64 (B,H,N) the leaf budgets, nL int32 (B,H,N) the distinct matched
+ * leaves (NULL: none), nid int32 and match (B,H,N,S) as ta_neighbor_pass writes them (S 0: none), tq int32 positions,
+ * tq[b * tq_sb + n].  Writes n_tree int32 (B,H,N) (the budget split; may be NULL), cm int32 (B,H,N,KC) with KC =
+ * (wl + S) * leaf + 1 + max(local, 3) (+ leaf when leaf > 2), entries in ta_assemble_candidates' order (may be NULL),
+ * and sums int32 (sum_rows, 5), the columns' sums over sum_rows parts of the rows: kept entries, kept tree entries,
+ * kept neighbour entries, leaves used, nL.  wl, S at most 64; leaf a power of two.
+ */
+int ta_assemble_leaves(const int32_t* ids, const uint8_t* vld, const int64_t* lhat, const int32_t* nL,
+                       const int32_t* nid, const uint8_t* match, const int32_t* tq, int64_t tq_sb, int B, int H,
+                       int N, int wl, int S, int leaf, int local, int wmax, int32_t* n_tree, int32_t* cm,
+                       int32_t* sums, int sum_rows, void* stream);
+
+
+/*
  * Softmax attention of each query over an explicit candidate list (replaces fastseg.py:173-177
  * sparse_attn forward, its kernel fastseg.py:50-78 and the fallback fastseg.py:134-141).
  * q: (B,H,T,D), k, v: (B,H,Tk,D), same dtype; cand: (B,H,T,KC) int32 contiguous, -1 = unused, duplicates

@@ -95,6 +95,7 @@ SIGNATURES = {
                                      c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_f32, c_vp, c_vp]),
     'ta_assemble_candidates': (c_i32, [c_vp, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32,
                                        c_i32, c_vp, c_vp, c_vp]),
+    'ta_assemble_leaves': (c_i32, [c_vp] * 7 + [c_i64] + [c_i32] * 8 + [c_vp, c_vp, c_vp, c_i32, c_vp]),
     'ta_sparse_attn_fwd': (c_i32, [c_vp, c_vp, c_vp, c_i32, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64,
                                    c_i64, c_i64, c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_f32, c_vp,
                                    c_vp, _P(KvPages), c_vp]),

@@ -763,16 +763,18 @@ class Decoder:
                     # own tree pass, which the selection's own neighbour pass reads too
                     if lhat is None:
                         lhat = torch.full((nb, H, T0), cfg.beam, dtype=torch.long, device=self.dev)
-                    sel, ids, vld, sct, _ = SEL.select(q, k, lhat, cfg, st.shape, lv)
-                    n = min(cfg.nb_store, ids.shape[-1])
-                    vb = vld[..., :n].bool()
-                    st.st_leaf[b0:b1, :, :T0, :n] = ids[..., :n].clamp(min=0)
-                    st.st_score[b0:b1, :, :T0, :n] = torch.where(vb, sct[..., :n], torch.zeros_like(sct[..., :n]))
-                    st.st_ok[b0:b1, :, :T0, :n] = vb
-                    cand, keep, _ = SEL.assemble(sel, tq.long(), cfg, nb, H)
-                    o, _ = K.sparse_attn_fwd(q, k, v, torch.where(keep, cand, torch.full_like(cand, -1)), scale)
+                    store = tuple(x[b0:b1, :, :T0] for x in (st.st_leaf, st.st_score, st.st_ok))
+                    ids, vld, sct, bor, _ = SEL.select_leaves(q, k, cfg, st.shape, lv, tq=tq, store=store)
+                    if K.leaves_supported(ids.shape[-1], st.shape.leaf, cfg.nb_window * cfg.nb_store, cfg.local):
+                        cm, _, _ = K.assemble_leaves(ids, vld, lhat, cfg, st.shape.leaf, tq, bor)
+                    else:
+                        sel = SEL.expand(ids, vld, bor, lhat, cfg, st.shape.leaf)
+                        cand, keep, _ = SEL.assemble(sel, tq.long(), cfg, nb, H)
+                        cm = torch.where(keep, cand, torch.full_like(cand, -1))
+                        del sel, cand, keep
+                    o, _ = K.sparse_attn_fwd(q, k, v, cm, scale)
                     out.transpose(1, 2).copy_(o)
-                    del sel, ids, vld, sct, cand, keep, o
+                    del ids, vld, sct, bor, cm, o
                 else:
                     # no neighbour borrowing: the tree leaves of each query's budget plus the static and local
                     # keys, attended by the structural kernel (the same key set as the candidate list, which at

@@ -196,9 +196,10 @@ class SegAttention(nn.Module):
         scale = 1.0 / math.sqrt(dh)
         self.aux = {}
         lhat, plog = self.budget(q, k)
-        out, aux, sel, ck = SEL.attend(q, k, v, lhat, cfg, scale)
+        losses = self.training and cfg.beam_mode == 'pred'
+        out, aux, sel, ck = SEL.attend(q, k, v, lhat, cfg, scale, want_sel=losses)
         self.aux.update({name: val.detach() for name, val in aux.items()})
-        if self.training and cfg.beam_mode == 'pred':
+        if losses:
             self.aux.update(self._pred_loss(q, k, sel, ck, plog, scale))
         return out
 

@@ -118,7 +118,11 @@ def level_sums(k, blevels, out=None, t_end=None, zero_sink=True, log_magnitudes=
     B, H, T, D = k.shape
     t_end = T if t_end is None else int(t_end)
     if out is None:
-        out = [torch.zeros(B, H, T >> l, D, device=k.device, dtype=torch.float32) for l in blevels]
+        # one buffer for all levels; every node is written when the keys are complete
+        alloc = torch.empty if t_end >= T else torch.zeros
+        rows = [T >> l for l in blevels]
+        buf = alloc(B * H * sum(rows) * D, device=k.device, dtype=torch.float32)
+        out = [p.view(B, H, n, D) for p, n in zip(buf.split([B * H * n * D for n in rows]), rows)]
     for o in out:
         if o.stride(-1) != 1 or o.stride(-2) != D:
             raise ValueError('level tensors need contiguous node rows')
@@ -581,6 +585,36 @@ def assemble_candidates(sel, tq, local, leaf, b, H):
     L.call('ta_assemble_candidates', L.ptr(tree_pos), L.ptr(leaf_ok), L.ptr(n_tree), L.ptr(nb_pos), L.ptr(tq),
            1 if tq.dim() == 2 else 0, b, H, N, wl, leaf, nbk, int(local), L.ptr(cm), L.ptr(counts), L.stream())
     return cm, counts
+
+
+def leaves_supported(wl, leaf, S, local):
+    """Whether assemble_leaves takes these widths."""
+    return 1 <= wl <= 64 and S <= 64 and max(local, 3) < 64
+
+
+def assemble_leaves(ids, vld, lhat, cfg, leaf, tq=None, nb=None, cand=True):
+    """The masked candidate list, the leaf budgets and the statistics' means from a selection's leaves in one launch
+    (ta_assemble_leaves): ids int32, vld uint8 (b,H,N,wl) of a descent, lhat (b,H,N) budgets, tq int32 (N,) or (b,N)
+    positions (only needed for the list), nb = (nid int32, match bool, nL int32) of neighbor_pass or None.  Returns
+    (cm (b,H,N,KC) int32 or None without `cand`, n_tree (b,H,N) int32, means (5,) float32: kept entries, kept tree
+    entries, kept neighbour entries, leaves used, matched leaves, per row)."""
+    b, H, N, wl = ids.shape
+    nid, match, nL = nb if nb is not None else (None, None, None)
+    S = nid.shape[-1] if nid is not None else 0
+    lh = lhat.to(torch.int64).contiguous()
+    L.require_gpu(ids, vld, lh, nid, match, nL, tq)
+    dev = ids.device
+    n_tree = torch.empty(b, H, N, dtype=torch.int32, device=dev)
+    cm = (torch.empty(b, H, N, candidate_width(wl, leaf, S * leaf, cfg.local), dtype=torch.int32, device=dev)
+          if cand else None)
+    rows = b * H * N
+    parts = max(1, min(1024, (rows + 7) // 8))
+    sums = torch.empty(parts, 5, dtype=torch.int32, device=dev)
+    L.call('ta_assemble_leaves', L.ptr(ids), L.ptr(vld), L.ptr(lh), L.ptr(nL), L.ptr(nid), L.ptr(match), L.ptr(tq),
+           tq.stride(0) if tq is not None and tq.dim() == 2 else 0, b, H, N, wl, S, int(leaf), int(cfg.local),
+           int(cfg.wmax), L.ptr(n_tree), L.ptr(cm), L.ptr(sums), parts, L.stream())
+    means = sums.sum(0, dtype=torch.float64).mul_(1.0 / rows).float()
+    return cm, n_tree, means
 
 
 def sparse_attn_fwd(q, k, v, cand, scale):

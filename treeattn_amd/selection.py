@@ -149,46 +149,68 @@ def assemble(sel, tq, cfg, b, H):
     return cand, keep, used
 
 
-def select(q, k, lhat, cfg, shape=None, levels=None):
-    """Whole-sequence selection (seg.py:122-140 / fastseg.py:302-314) on the device.  `levels`: the levels the
-    selection scores, already built for `shape` (a decode cache's: gated where the gate applies), else they are
-    built from k (with the gate when cfg.gate).  Returns (sel dict, ids, vld, sct, levels)."""
+def select_leaves(q, k, cfg, shape=None, levels=None, tq=None, store=None):
+    """The leaves of a whole-sequence selection (seg.py:122-140 / fastseg.py:302-314) as the kernels write them:
+    (ids int32, vld uint8, sct float32 (b,H,T,wl), nb, levels) with nb = (nid int32, match bool, nL int32) of the
+    neighbour pass, or None without neighbour borrowing.  `levels`: the levels the selection scores, already built
+    for `shape` (a decode cache's: gated where the gate applies), else they are built from k (with the gate when
+    cfg.gate).  store: (st_leaf, st_score, st_ok) arrays (b,H,T,nb_store) to keep the stored leaves in (a decode
+    cache's, their slots past the found leaves left alone)."""
     check_supported(cfg)
     b, H, T, dh = q.shape
     shape = shape or cfg_shape(cfg, T)
     if levels is None:
         levels = build_gated(k, shape, build_pyramid(k, shape), cfg)
-    tq = torch.arange(T, device=q.device)
-    ids32, vld8, sct = K.tree_descend(q, levels, tq, shape, cfg.wmax)
-    ids, vld = ids32.long(), vld8.bool()
+    if tq is None:
+        tq = torch.arange(T, device=q.device, dtype=torch.int32)
     NS = cfg.nb_store
-    wl = ids.shape[-1]
-    if cfg.neighbors and shape.n_levels > 0:
-        n = min(NS, wl)
-        st_leaf = torch.zeros(b, H, T, NS, dtype=torch.int32, device=q.device)
-        st_score = torch.zeros(b, H, T, NS, device=q.device)
-        st_ok = torch.zeros(b, H, T, NS, dtype=torch.bool, device=q.device)
-        st_leaf[..., :n] = ids32[..., :n].clamp(min=0)
-        st_score[..., :n] = torch.where(vld[..., :n], sct[..., :n], torch.zeros_like(sct[..., :n]))
-        st_ok[..., :n] = vld[..., :n]
-        nid, match, nL = neighbor_pass(q.float(), levels[0], st_leaf, st_score, st_ok, tq, cfg, shape.leaf)
+    wl = shape.leaf_width(cfg.wmax)
+    if not cfg.neighbors or shape.n_levels == 0:
+        ids, vld, sct = K.tree_descend(q, levels, tq, shape, cfg.wmax)
+        return ids, vld, sct, None, levels
+    n = min(NS, wl)
+    if store is None:   # every slot is written by the descent unless a row holds fewer leaves than it stores
+        alloc = torch.empty if n == NS else torch.zeros
+        store = tuple(alloc(b, H, T, NS, dtype=d, device=q.device) for d in (torch.int32, torch.float32, torch.bool))
+    ids, vld, sct = K.tree_descend(q, levels, tq, shape, cfg.wmax, store=(*store, n))
+    nb = K.neighbor_pass(q, levels[0], *store, tq, cfg, shape.leaf)
+    return ids, vld, sct, nb, levels
+
+
+def expand(ids32, vld8, nb, lhat, cfg, leaf):
+    """The reference's selection dict (seg.py:106-119) of select_leaves' results."""
+    b, H, T, wl = ids32.shape
+    ids, vld = ids32.long(), vld8.bool()
+    if nb is not None:
+        nid, match, nL = nb[0].long(), nb[1], nb[2].long()
     else:
-        Wn = cfg.nb_window
-        nid = torch.zeros(b, H, T, Wn * NS, dtype=torch.long, device=q.device)
-        match = torch.zeros(b, H, T, Wn * NS, dtype=torch.bool, device=q.device)
-        nL = torch.zeros(b, H, T, dtype=torch.long, device=q.device)
-    sel = finish(torch.where(vld, ids, torch.zeros_like(ids)), vld, nid, match, nL, lhat, cfg, shape.leaf)
-    return sel, ids32, vld8, sct, levels
+        S = cfg.nb_window * cfg.nb_store
+        nid = torch.zeros(b, H, T, S, dtype=torch.long, device=ids.device)
+        match = torch.zeros(b, H, T, S, dtype=torch.bool, device=ids.device)
+        nL = torch.zeros(b, H, T, dtype=torch.long, device=ids.device)
+    return finish(torch.where(vld, ids, torch.zeros_like(ids)), vld, nid, match, nL, lhat, cfg, leaf)
 
 
-def attend(q, k, v, lhat, cfg, scale=None):
-    """SegAttention.sparse_attend without its budget head: returns (out, aux, used, keep-or-None).
-    Neighbours off and a fixed budget use the structural kernel (no candidate list); otherwise the
-    candidate list of the reference is built and attended by the candidate-list kernel."""
+def select(q, k, lhat, cfg, shape=None, levels=None):
+    """Whole-sequence selection (seg.py:122-140 / fastseg.py:302-314) on the device; `levels` as in select_leaves.
+    Returns (sel dict, ids, vld, sct, levels)."""
+    shape = shape or cfg_shape(cfg, q.shape[2])
+    ids, vld, sct, nb, levels = select_leaves(q, k, cfg, shape, levels)
+    return expand(ids, vld, nb, lhat, cfg, shape.leaf), ids, vld, sct, levels
+
+
+def attend(q, k, v, lhat, cfg, scale=None, want_sel=True):
+    """SegAttention.sparse_attend without its budget head: returns (out, aux, sel dict, keep-or-None).
+    Neighbours off without gradients use the structural kernel (no candidate list); otherwise the candidate list of
+    the reference is built and attended by the candidate-list kernel.  want_sel=False leaves the selection dict out
+    (None) where the attention does not need it: its expanded positions are as large as the keys they name."""
     b, H, T, dh = q.shape
     scale = 1.0 / math.sqrt(dh) if scale is None else scale
-    tq = torch.arange(T, device=q.device)
-    if getattr(cfg, 'attn', 'seg') == 'dyn':   # the LaneTree selection (attention_dyn.py:74-75)
+    dyn = getattr(cfg, 'attn', 'seg') == 'dyn'
+    # gradients wanted (training): the candidate-list kernels, whose backward is built (the structural kernel
+    # attends the same key set, forward only)
+    grad = torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v))
+    if dyn:   # the LaneTree selection (attention_dyn.py:74-75)
         from .dyntree import select_keys
         leaf = 2
         sel = select_keys(q.detach(), k.detach(), lhat, cfg)
@@ -196,42 +218,54 @@ def attend(q, k, v, lhat, cfg, scale=None):
     else:
         shape = cfg_shape(cfg, T)
         leaf = shape.leaf
-        sel, ids32, vld8, sct, levels = select(q.detach(), k.detach(), lhat, cfg, shape)
-        wl = ids32.shape[-1]
+        tq32 = torch.arange(T, device=q.device, dtype=torch.int32)
+        ids, vld, _, nb, _ = select_leaves(q.detach(), k.detach(), cfg, shape, tq=tq32)
+        wl = ids.shape[-1]
+        S = cfg.nb_window * cfg.nb_store if nb is not None else 0
+        structural = not cfg.neighbors and not grad
+        if K.leaves_supported(wl, leaf, S, cfg.local):
+            # the candidate list, the budgets and the statistics from the leaves in one launch
+            cm, n_tree, m = K.assemble_leaves(ids, vld, lhat, cfg, leaf, tq32, nb, cand=not structural)
+            if structural:
+                keys = torch.empty(b, H, T, device=q.device)
+                out, _, keys = K.seg_attn(q, k, v, tq32, ids, vld, n_tree, leaf, cfg.local, scale, keys=keys)
+                aux = dict(keys_total=keys.mean(), keys_tree=m[3] * leaf, keys_nb=m[2], nb_leaves=m[4],
+                           leaves_used=m[3])
+            else:
+                out = _attend_list(q, k, v, cm, scale, grad)
+                aux = dict(keys_total=m[0], keys_tree=m[1], keys_nb=m[2], nb_leaves=m[4], leaves_used=m[3])
+            return out, aux, expand(ids, vld, nb, lhat, cfg, leaf) if want_sel else None, None
+        sel = expand(ids, vld, nb, lhat, cfg, leaf)
+        if structural:
+            n_tree = sel['n_tree'].to(torch.int32)
+            keys = torch.empty(b, H, T, device=q.device)
+            out, _, keys = K.seg_attn(q, k, v, tq32, ids, vld, n_tree, leaf, cfg.local, scale, keys=keys)
+            used = vld.bool() & (torch.arange(wl, device=q.device) < n_tree.unsqueeze(-1))
+            nused = used.sum(-1).float()
+            aux = dict(keys_total=keys.mean(), keys_tree=(nused * leaf).mean(),
+                       keys_nb=torch.zeros((), device=q.device), nb_leaves=sel['nb_leaves'].float().mean(),
+                       leaves_used=nused.mean())
+            return out, aux, sel, None
+    tq = torch.arange(T, device=q.device)
     NBK = sel['nb_pos'].shape[-1]
-    # gradients wanted (training): the candidate-list kernels, whose backward is built (the structural kernel
-    # attends the same key set, forward only)
-    grad = torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v))
-    if not cfg.neighbors and not grad and getattr(cfg, 'attn', 'seg') != 'dyn':
-        n_tree = sel['n_tree'].to(torch.int32)
-        keys = torch.empty(b, H, T, device=q.device)
-        out, _, keys = K.seg_attn(q, k, v, tq, ids32, vld8, n_tree, leaf, cfg.local, scale, keys=keys)
-        used = vld8.bool() & (torch.arange(wl, device=q.device) < n_tree.unsqueeze(-1))
-        nused = used.sum(-1).float()
-        aux = dict(keys_total=keys.mean(), keys_tree=(nused * leaf).mean(),
-                   keys_nb=torch.zeros((), device=q.device), nb_leaves=sel['nb_leaves'].float().mean(),
-                   leaves_used=nused.mean())
-        return out, aux, sel, None
     if K.candidate_width(wl, leaf, NBK, cfg.local) <= K.CAND_MAX:
         # the masked candidate list and its counts in one launch (the same list and statistics as below)
         cm, counts = K.assemble_candidates(sel, tq, cfg.local, leaf, b, H)
-        if grad:
-            from . import fastseg as FS
-            out = FS.sparse_attn(q, k, v, cm, scale, causal=True)
-        else:
-            out, _ = K.sparse_attn_fwd(q, k, v, cm, scale)
         c = counts.float().mean((0, 1, 2))
         aux = dict(keys_total=c[0], keys_tree=c[1], keys_nb=c[2], nb_leaves=sel['nb_leaves'].float().mean(),
                    leaves_used=c[3])
-        return out, aux, sel, None
+        return _attend_list(q, k, v, cm, scale, grad), aux, sel, None
     cand, keep, used = assemble(sel, tq, cfg, b, H)
     cm = torch.where(keep, cand, torch.full_like(cand, -1))
-    if grad:
-        from . import fastseg as FS
-        out = FS.sparse_attn(q, k, v, cm, scale, causal=True)
-    else:
-        out, _ = K.sparse_attn_fwd(q, k, v, cm, scale)
+    out = _attend_list(q, k, v, cm, scale, grad)
     aux = dict(keys_total=keep.sum(-1).float().mean(), keys_tree=keep[..., :leaf * wl].sum(-1).float().mean(),
                keys_nb=keep[..., leaf * wl:leaf * wl + NBK].sum(-1).float().mean(),
                nb_leaves=sel['nb_leaves'].float().mean(), leaves_used=used.sum(-1).float().mean())
     return out, aux, sel, (cand, keep)
+
+
+def _attend_list(q, k, v, cm, scale, grad):
+    if grad:
+        from . import fastseg as FS
+        return FS.sparse_attn(q, k, v, cm, scale, causal=True)
+    return K.sparse_attn_fwd(q, k, v, cm, scale)[0]

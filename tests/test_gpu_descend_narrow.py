@@ -1,0 +1,52 @@
+"""The descent of many queries with a beam of at most 8 over a binary tree (a 16-lane group per query) against the
+oracle's canonical descent, bit for bit.  GPU only."""
+import pytest
+import torch
+
+from oracle import seg_ref as S
+from treeattn_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda'
+
+
+@pytest.mark.parametrize('T,D,leaf,wmax,Nq,dtype', [
+    (1024, 64, 2, 8, 257, torch.float16),     # the fewest queries; a last group of one query
+    (4096, 128, 2, 8, 300, torch.float32),    # candidate rows in three parts
+    (512, 16, 2, 1, 512, torch.bfloat16),     # a beam of one
+    (256, 32, 2, 5, 256, torch.float32),      # every position, an odd beam
+    (64, 64, 32, 8, 64, torch.bfloat16),      # one level
+    (2048, 64, 16, 7, 1000, torch.bfloat16),
+])
+def test_narrow_descent_matches_oracle(T, D, leaf, wmax, Nq, dtype):
+    print('case', T, D, leaf, wmax, Nq, dtype, flush=True)
+    B, H = (3, 2) if Nq < 300 else (1, 2)
+    g = torch.Generator().manual_seed(T + D + wmax)
+    q = torch.randn(B, H, Nq, D, generator=g).to(dtype)
+    k = torch.randn(B, H, T, D, generator=g).to(dtype)
+    k[:, :, T // 2:] = k[:, :, :T // 2]       # repeated keys: equal scores, ranked by node id
+    # sorted positions from 0 on, some repeated, the last one included: starts differ within a wavefront
+    tq = torch.arange(T) if Nq == T else torch.sort(torch.randint(0, T, (Nq,), generator=g)).values
+    tq[-1] = T - 1
+    geom = S.Geometry(T, leaf, 2)
+    want = S.tree_pass_general(q.float(), S.pyramid(S.index_keys(k), geom), tq, geom, wmax, 'canonical')
+    shape = K.TreeShape(T, leaf, 2)
+    lv = K.level_sums(k.to(DEV), shape.blevels)
+    NS = 3
+    store = (torch.full((B, H, T, NS), -7, dtype=torch.int32, device=DEV), torch.full((B, H, T, NS), 7.0, device=DEV),
+             torch.ones(B, H, T, NS, dtype=torch.bool, device=DEV))
+    n = min(NS, shape.leaf_width(wmax))
+    ids, vld, sct = (x.cpu() for x in K.tree_descend(q.to(DEV), lv, tq.to(DEV), shape, wmax, store=(*store, n)))
+    ok = want[1]
+    assert torch.equal(vld.bool(), ok)
+    assert torch.equal(ids.long()[ok], want[0][ok]) and torch.equal(sct[ok], want[2][ok])
+    assert bool((ids[~ok] == -1).all())
+    sl, ss, so = (x.cpu() for x in store)
+    rows = tq.unique()                        # a repeated position is written by any of its (different) queries
+    once = [int(i) for i in rows if int((tq == i).sum()) == 1]
+    at = torch.tensor([int((tq == i).nonzero()[0]) for i in once])
+    w_ok = ok[:, :, at, :n]
+    assert torch.equal(so[:, :, once, :n], w_ok)
+    assert torch.equal(sl[:, :, once, :n].long(), torch.where(w_ok, want[0][:, :, at, :n], 0))
+    assert torch.equal(ss[:, :, once, :n], torch.where(w_ok, want[2][:, :, at, :n], 0.0))
+    assert bool((sl[..., n:] == -7).all())

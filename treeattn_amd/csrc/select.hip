@@ -321,6 +321,128 @@ __global__ __launch_bounds__(WPQ == 16 ? 1024 : 256) void descend_kernel(
   }
 }
 
+// Descent of many queries with a beam of at most 8 over a binary tree (17 candidates a level at most): a 16-lane group
+// per query, four queries per wavefront.  At that width the one-wavefront-per-query kernel is bound by its own
+// bookkeeping (about 300 instructions per level for 17 scores).  Here a level's candidate rows are all requested at
+// once, every lane of the group gets every score from the canonical dot's butterfly, lane c keeps candidate c (the
+// seventeenth is known to all), the ranks are counted with row rotations, and only the kept ids go through LDS.
+// Same scores, ranks and outputs.  (2, 6, 4096, 64) float16 over pairs of keys: 77 us against 300 us; (8, 6,
+// 512, 64) float32 29 against 100 us.
+constexpr int kNarrowW = 8;
+
+template <typename TQ, int D>
+__global__ __launch_bounds__(256) void descend_narrow_kernel(
+    const TQ* __restrict__ q, int64_t qsb, int64_t qsh, int64_t qsn, int H, int Nq, int T,
+    const int32_t* __restrict__ tq, int64_t tq_sb, LevelIn lv, int n_levels, int wmax, int wl,
+    int32_t* __restrict__ ids, uint8_t* __restrict__ vld, float* __restrict__ sct, ta_leaf_store_out so) {
+  constexpr int R = D / 16;
+  constexpr int NB = R >= 8 ? 6 : 17;   // candidate rows in flight (all, or a third of them at D = 128)
+  __shared__ __align__(16) int32_t s_kid[16][kNarrowW];
+  __shared__ float s_ksc[16][kNarrowW];
+  const int lane = lane_id(), w = wave_id();
+  const int g = lane >> 4, j16 = lane & 15;
+  int32_t* kid = s_kid[4 * w + g];
+  float* ksc = s_ksc[4 * w + g];
+  const int nn = (blockIdx.x * 4 + w) * 4 + g;
+  const bool live = nn < Nq;
+  const int n = live ? nn : Nq - 1;
+  const int bh = blockIdx.y;
+  const int b = bh / H, h = bh % H;
+  const int t = tq[b * tq_sb + n];
+  float qr[R];
+  load_row<TQ, R>(q + b * qsb + h * qsh + n * qsn + R * j16, qr);
+  int start = -1;
+  if (t > 0 && t < T) {
+    for (int j = n_levels - 1; j >= 0; --j) {
+      if (start < 0 && ((t >> lv.blevel[j]) > wmax || j == 0)) start = j;
+    }
+  }
+  if (j16 < kNarrowW) kid[j16] = 0;
+  wave_sync();
+  int nk = 0;
+  for (int j = n_levels - 1; j >= 0; --j) {
+    const bool on = j <= start;
+    if (!__any(on)) continue;
+    const bool first = j == start;
+    const int m = t >> lv.blevel[j];
+    const int nch = first ? (m < 16 ? m : 16) : 2 * nk;          // candidates 0 .. nch - 1 of the sixteen
+    const bool xv = on && (first ? m > 16 : (m & 1) != 0);      // the seventeenth: the last node, or the left sibling
+    const int xid = first ? 16 : m - 1;
+    const int4 ka = *reinterpret_cast<const int4*>(kid), kb = *reinterpret_cast<const int4*>(kid + 4);
+    const int kept[kNarrowW] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
+    const int mine_id = first ? j16 : 2 * kid[j16 >> 1] + (j16 & 1);
+    const float* base = lv.ptr[j] + b * lv.sb[j] + h * lv.sh[j] + R * j16;
+    const float scale = pow2_neg(lv.blevel[j]);
+    float mine = 0.0f, xs = 0.0f;
+#pragma unroll
+    for (int c0 = 0; c0 < 17; c0 += NB) {
+      float rows[NB][R];
+#pragma unroll
+      for (int r = 0; r < NB; ++r) {
+        const int c = c0 + r;
+        if (c < 17) {
+          const int id = c == 16 ? (xv ? xid : 0) : (on && c < nch ? (first ? c : 2 * kept[c >> 1] + (c & 1)) : 0);
+          load_row_g<float, R>(base + (int64_t)id * D, rows[r]);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < NB; ++r) {
+        const int c = c0 + r;
+        if (c < 17) {
+          const float s = __fmul_rn(canon_dot<R>(qr, rows[r]), scale);
+          if (c == 16) xs = s;
+          else if (j16 == c) mine = s;
+        }
+      }
+    }
+    const bool mv = on && j16 < nch;
+    const uint64_t key = mv ? rank_key(mine, mine_id) : 0;
+    const uint64_t xkey = xv ? rank_key(xs, xid) : 0;
+    int rank = xkey > key ? 1 : 0;
+    const int klo = (int)(uint32_t)key, khi = (int)(uint32_t)(key >> 32);
+    auto against = [&](int lo, int hi) {
+      rank += ((uint64_t)(uint32_t)hi << 32 | (uint32_t)lo) > key ? 1 : 0;
+    };
+#define TA_ROT(N)                                                                  \
+  against(__builtin_amdgcn_update_dpp(0, klo, 0x120 + N, 0xF, 0xF, false),         \
+          __builtin_amdgcn_update_dpp(0, khi, 0x120 + N, 0xF, 0xF, false))
+    TA_ROT(1); TA_ROT(2); TA_ROT(3); TA_ROT(4); TA_ROT(5); TA_ROT(6); TA_ROT(7); TA_ROT(8);
+    TA_ROT(9); TA_ROT(10); TA_ROT(11); TA_ROT(12); TA_ROT(13); TA_ROT(14); TA_ROT(15);
+#undef TA_ROT
+    const int xrank = __popc((uint32_t)(__ballot(key > xkey) >> (16 * g)) & 0xFFFFu);
+    wave_sync();   // every lane has read the kept ids
+    if (mv && rank < wmax) {
+      kid[rank] = mine_id;
+      ksc[rank] = mine;
+    }
+    if (xv && j16 == 0 && xrank < wmax) {
+      kid[xrank] = xid;
+      ksc[xrank] = xs;
+    }
+    if (on) {
+      const int C = nch + (xv ? 1 : 0);
+      nk = C < wmax ? C : wmax;
+    }
+    wave_sync();
+  }
+  if (!live) return;
+  const int64_t obase = ((int64_t)bh * Nq + n) * wl;
+  if (j16 < wl) {
+    const bool ok = j16 < nk;
+    ids[obase + j16] = ok ? kid[j16] : -1;
+    vld[obase + j16] = ok ? 1 : 0;
+    sct[obase + j16] = ok ? ksc[j16] : -INFINITY;
+  }
+  if (so.leaf != nullptr && t >= 0 && t < so.Tst && j16 < so.n) {
+    // the neighbour store of position t: kept leaves first, empty slots as id 0, score 0, not ok
+    const int64_t sbase = b * so.sb + h * so.sh + (int64_t)t * so.st;
+    const bool ok = j16 < nk;
+    so.leaf[sbase + j16] = ok ? max(kid[j16], 0) : 0;
+    so.score[sbase + j16] = ok ? ksc[j16] : 0.0f;
+    so.ok[sbase + j16] = ok ? 1 : 0;
+  }
+}
+
 // ----------------------------------------------------------------------------------------- gather-dot
 // One wavefront per query row; 4 candidates per round (16 lanes each).  blk != nullptr selects the
 // leaf-block form: candidate c is row blk[c >> block_log2] * block + (c & (block - 1)).
@@ -506,6 +628,14 @@ struct DescendRun {
   hipLaunchKernelGGL((descend_kernel<T, D, WPQ, APP, GT>), grid, dim3(NTH), lds, st, (const T*)q, qsb, qsh, qsn, H, \
                      Nq, Tgeo, tq, tq_sb, lv, n_levels, arity_log2, wmax, wl, cmax4, ids, vld, sct,                  \
                      ap ? *ap : none, alv ? *alv : lv, so ? *so : no_store, ga ? *ga : no_gate)
+    // a beam of at most 8 over a binary tree: a 16-lane group per query (wl never exceeds the beam).  From 257
+    // queries on: against four wavefronts per query 39 -> 20 us at (1, 6, 512, 64), against one 300 -> 77 us at (2, 6,
+    // 4096, 64), 655 -> 148 us at (2, 12, 8192, 64) over leaves of 32; up to 256 both take what a launch takes.
+    if (!ap && arity_log2 == 1 && wmax <= kNarrowW && wl <= kNarrowW && nq_all > 256) {
+      hipLaunchKernelGGL((descend_narrow_kernel<T, D>), dim3((Nq + 15) / 16, B * H), dim3(256), 0, st, (const T*)q, qsb,
+                         qsh, qsn, H, Nq, Tgeo, tq, tq_sb, lv, n_levels, wmax, wl, ids, vld, sct, so ? *so : no_store);
+      return check_launch("descend_narrow_kernel");
+    }
     if (ap && ga) {
       if (wpq == 16) TA_DESC(16, 1024, true, true);
       else TA_DESC(4, 256, true, true);

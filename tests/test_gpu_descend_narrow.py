@@ -1,5 +1,5 @@
-"""The descent of many queries with a beam of at most 8 over a binary tree (a 16-lane group per query) against the
-oracle's canonical descent, bit for bit.  GPU only."""
+"""The two forms of the descent of many queries -- a beam of at most 8 over a binary tree (a 16-lane group per query), and
+wide beams whose kept set is found without ranking -- against the oracle's canonical descent, bit for bit.  GPU only."""
 import pytest
 import torch
 
@@ -50,3 +50,26 @@ def test_narrow_descent_matches_oracle(T, D, leaf, wmax, Nq, dtype):
     assert torch.equal(sl[:, :, once, :n].long(), torch.where(w_ok, want[0][:, :, at, :n], 0))
     assert torch.equal(ss[:, :, once, :n], torch.where(w_ok, want[2][:, :, at, :n], 0.0))
     assert bool((sl[..., n:] == -7).all())
+
+
+@pytest.mark.parametrize('T,D,leaf,arity,wmax,copies', [
+    (8192, 64, 32, 2, 32, 1),      # 64 and 65 candidates
+    (8192, 64, 32, 2, 32, 16),     # equal scores at the border of the kept set
+    (2048, 16, 16, 4, 31, 1),      # up to 127 candidates, a beam that is no multiple of 4
+    (4096, 32, 32, 2, 64, 4),      # 128 and 129 candidates: both sides of what one wavefront holds
+])
+def test_wide_descent_matches_oracle(T, D, leaf, arity, wmax, copies):
+    print('case', T, D, leaf, arity, wmax, copies, flush=True)
+    B, H, Nq = 1, 2, 2200
+    g = torch.Generator().manual_seed(T + D + wmax)
+    q = torch.randn(B, H, Nq, D, generator=g)
+    k = torch.randn(B, H, T // copies, D, generator=g).repeat(1, 1, copies, 1)
+    tq = torch.sort(torch.randint(0, T, (Nq,), generator=g)).values
+    geom = S.Geometry(T, leaf, arity)
+    want = S.tree_pass_general(q, S.pyramid(S.index_keys(k), geom), tq, geom, wmax, 'canonical')
+    shape = K.TreeShape(T, leaf, arity)
+    lv = K.level_sums(k.to(DEV), shape.blevels)
+    ids, vld, sct = (x.cpu() for x in K.tree_descend(q.to(DEV), lv, tq.to(DEV), shape, wmax))
+    ok = want[1]
+    assert torch.equal(vld.bool(), ok)
+    assert torch.equal(ids.long()[ok], want[0][ok]) and torch.equal(sct[ok], want[2][ok])

@@ -90,14 +90,77 @@ __device__ __forceinline__ int quad_xor(int x) {
   return __builtin_amdgcn_update_dpp(0, x, ctrl, 0xF, 0xF, false);
 }
 
+// The wmax best of C candidates (wmax < C <= 128; one wavefront, candidates lane and lane + 64 of ckey / cid / csc)
+// without ranking them: the wmax-th largest key is found bit by bit from the top with ballots (it usually ends within
+// about fifteen steps, when exactly wmax keys are at or above the trial value), where counting every rank reads every
+// key in every lane, twice for the sixty-fifth candidate.  Above the leaf level the order of the kept nodes does not
+// matter: their ids are left in kid and 0 is returned.  At the leaf level the kept candidates are moved to the front
+// of ckey / cid / csc (padded to a multiple of 4 as the ranking reads them) and wmax is returned.
+__device__ __forceinline__ int keep_best(int C, int wmax, int lane, bool inner, uint64_t* ckey, int32_t* cid, float* csc,
+                                         int32_t* kid) {
+  const bool in1 = lane + kWave < C;
+  const uint64_t k0 = lane < C ? ckey[lane] : 0, k1 = in1 ? ckey[lane + kWave] : 0;
+  const uint32_t h0 = (uint32_t)(k0 >> 32), h1 = (uint32_t)(k1 >> 32);
+  uint32_t v = 0;
+  int n = 0;
+  for (int bit = 31; bit >= 0 && n != wmax; --bit) {
+    const uint32_t trial = v | (1u << bit);
+    const int m = __popcll(__ballot(h0 >= trial)) + __popcll(__ballot(h1 >= trial));
+    if (m >= wmax) {
+      v = trial;
+      n = m;
+    }
+  }
+  bool keep0 = h0 >= v && lane < C, keep1 = h1 >= v && in1;
+  if (n != wmax) {   // equal scores at the border: of those, the lowest ids (the larger low words)
+    const bool e0 = h0 == v && lane < C, e1 = h1 == v && in1;
+    keep0 = h0 > v && lane < C;
+    keep1 = h1 > v && in1;
+    const int need = wmax - __popcll(__ballot(keep0)) - __popcll(__ballot(keep1));
+    const uint32_t l0 = (uint32_t)k0, l1 = (uint32_t)k1;
+    uint32_t u = 0;
+    for (int bit = 30; bit >= 0; --bit) {
+      const uint32_t trial = u | (1u << bit);
+      const int m = __popcll(__ballot(e0 && l0 >= trial)) + __popcll(__ballot(e1 && l1 >= trial));
+      if (m >= need) u = trial;
+    }
+    keep0 = keep0 || (e0 && l0 >= u);
+    keep1 = keep1 || (e1 && l1 >= u);
+  }
+  const uint64_t below = (1ull << lane) - 1, m0 = __ballot(keep0), m1 = __ballot(keep1);
+  const int p0 = __popcll(m0 & below), p1 = __popcll(m0) + __popcll(m1 & below);
+  const int i0 = lane < C ? cid[lane] : 0, i1 = in1 ? cid[lane + kWave] : 0;
+  if (inner) {
+    if (keep0) kid[p0] = i0;
+    if (keep1) kid[p1] = i1;
+    return 0;
+  }
+  const float s0 = lane < C ? csc[lane] : 0.0f, s1 = in1 ? csc[lane + kWave] : 0.0f;
+  wave_sync();   // every lane has read its candidates
+  if (keep0) {
+    ckey[p0] = k0;
+    cid[p0] = i0;
+    csc[p0] = s0;
+  }
+  if (keep1) {
+    ckey[p1] = k1;
+    cid[p1] = i1;
+    csc[p1] = s1;
+  }
+  if (lane < 4 && wmax + lane < ((wmax + 3) & ~3)) ckey[wmax + lane] = 0;
+  wave_sync();
+  return wmax;
+}
+
 // One query at position t: WPQ wavefronts (threads tid = 0 .. 64 WPQ - 1 of the query group) descend the
 // levels of lv for the tree of geometry T and leave the kept leaf-level nodes, best first, in kid / ksc
 // (LDS); returns how many there are (at most wmax).  qrow: the query's D elements (any address space).
+// SEL: wide candidate lists are cut to the kept set before they are ranked (keep_best).
 // LDS per query: ckey[cmax4] (uint64), cid[cmax4], csc[cmax4], kid[wmax4], ksc[wmax4].
 // ptrow (paged caches, else null): the query's page table row; the pages of the leaf-level candidates are
 // copied into LDS (cpg[cmax4 rounded up to 64]) while their node rows load, and the kept leaves' pages left in
 // kpg[wmax4], so an attention that follows needs no further round trip to the table.
-template <typename TQ, int D, int WPQ>
+template <typename TQ, int D, int WPQ, bool SEL = false>
 __device__ __forceinline__ int descend_query(const TQ* qrow, int t, int T, int b, int h, const LevelIn& lv,
                                              int n_levels, int arity_log2, int wmax, int tid, uint64_t* ckey,
                                              int32_t* cid, float* csc, int32_t* kid, float* ksc,
@@ -172,8 +235,16 @@ __device__ __forceinline__ int descend_query(const TQ* qrow, int t, int T, int b
       if (ptrow != nullptr && j == 0 && tid < kWave) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       query_sync<WPQ>();
       TA_DMARK(1 + 2 * lvl_done);
+      int Cr = C;   // candidates left to rank
+      if constexpr (SEL) {
+        static_assert(WPQ == 1, "one wavefront keeps the candidates");
+        // at the leaf level the kept ones are ranked all the same, which one round of lanes does for up to 64
+        if (C > wmax && C > (j > 0 ? 40 : kWave) && C <= 2 * kWave && ptrow == nullptr)
+          Cr = keep_best(C, wmax, tid, j > 0, ckey, cid, csc, kid);
+      }
       // rank = number of candidates with a larger key; P lanes (a quad's aligned part) share a candidate
-      {
+      if (Cr > 0) {
+        const int C = Cr;
         const int C2 = (C + 1) >> 1;
         const int P = 4 * C <= NT ? 4 : (2 * C <= NT ? 2 : 1);
         const int lp = P == 4 ? 2 : P - 1;

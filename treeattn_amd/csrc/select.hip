@@ -247,7 +247,7 @@ struct DescentGateView {
 
 // Descent of one query per WPQ wavefronts; with APPEND (one query per (sequence, head)) the decode-cache
 // append of ap (rows of the query's element type) runs in the same launch.
-template <typename TQ, int D, int WPQ, bool APPEND, bool GATE>
+template <typename TQ, int D, int WPQ, bool APPEND, bool GATE, bool SEL = false>
 __global__ __launch_bounds__(WPQ == 16 ? 1024 : 256) void descend_kernel(
     const TQ* __restrict__ q, int64_t qsb, int64_t qsh, int64_t qsn, int H, int Nq, int T,
     const int32_t* __restrict__ tq, int64_t tq_sb, LevelIn lv, int n_levels, int arity_log2, int wmax, int wl,
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(WPQ == 16 ? 1024 : 256) void descend_kernel(
   }
   TA_DMARK(13);
   const int64_t obase = ((int64_t)bh * Nq + n) * wl;
-  const int nk = descend_query<TQ, D, WPQ>(q + b * qsb + h * qsh + n * qsn, t, T, b, h, lv, n_levels, arity_log2,
+  const int nk = descend_query<TQ, D, WPQ, SEL>(q + b * qsb + h * qsh + n * qsn, t, T, b, h, lv, n_levels, arity_log2,
                                            wmax, tid, ckey, cid, csc, kid, ksc);
   TA_DMARK(14);
   for (int r = tid; r < wl; r += NT) {
@@ -624,10 +624,11 @@ struct DescendRun {
     const AppendIn none{};
     const ta_leaf_store_out no_store{};
     const GateAppendIn no_gate{};
-#define TA_DESC(WPQ, NTH, APP, GT)                                                                                \
-  hipLaunchKernelGGL((descend_kernel<T, D, WPQ, APP, GT>), grid, dim3(NTH), lds, st, (const T*)q, qsb, qsh, qsn, H, \
+#define TA_DESC_S(WPQ, NTH, APP, GT, SEL)                                                                                \
+  hipLaunchKernelGGL((descend_kernel<T, D, WPQ, APP, GT, SEL>), grid, dim3(NTH), lds, st, (const T*)q, qsb, qsh, qsn, H, \
                      Nq, Tgeo, tq, tq_sb, lv, n_levels, arity_log2, wmax, wl, cmax4, ids, vld, sct,                  \
                      ap ? *ap : none, alv ? *alv : lv, so ? *so : no_store, ga ? *ga : no_gate)
+#define TA_DESC(WPQ, NTH, APP, GT) TA_DESC_S(WPQ, NTH, APP, GT, false)
     // a beam of at most 8 over a binary tree: a 16-lane group per query (wl never exceeds the beam).  From 257
     // queries on: against four wavefronts per query 39 -> 20 us at (1, 6, 512, 64), against one 300 -> 77 us at (2, 6,
     // 4096, 64), 655 -> 148 us at (2, 12, 8192, 64) over leaves of 32; up to 256 both take what a launch takes.
@@ -645,9 +646,14 @@ struct DescendRun {
     } else {
       if (wpq == 16) TA_DESC(16, 1024, false, false);
       else if (wide) TA_DESC(4, 256, false, false);
+      // wide lists cut before they are ranked: 65 candidates 3.94 -> 3.58 ms (4, 16, 16384, 128) and 766 -> 727 us
+      // (3, 12, 8192, 64), 131 candidates 296 -> 262 us.  Up to 40 candidates, or 64 leaves before the last query
+      // (positions usually run to Nq), counting the ranks is the faster: 434 against 486 us at 33 candidates.
+      else if (arity * wmax + arity - 1 > 40 && (Nq >> lv.blevel[0]) > kWave) TA_DESC_S(1, 256, false, false, true);
       else TA_DESC(1, 256, false, false);
     }
 #undef TA_DESC
+#undef TA_DESC_S
     return check_launch("descend_kernel");
   }
 };

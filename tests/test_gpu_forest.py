@@ -224,3 +224,21 @@ def test_attention_gradients_match_oracle():
     (got * g.to(DEV)).sum().backward()
     for a, b in ((qd, qs), (kd, ks), (vd, vs)):
         assert (a.grad.cpu() - b.grad).abs().max().item() < 1e-4
+
+
+@pytest.mark.parametrize('D,dtype', [(16, torch.float32), (64, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize('nb,block,wmax,bq', [(1, 8, 8, 8), (2, 4, 1, 1), (3, 4, 8, 5), (17, 4, 5, 5), (33, 8, 8, 3),
+                                              (48, 4, 7, 8), (70, 16, 8, 8)])
+def test_narrow_descent_equals_wide(D, dtype, nb, block, wmax, bq):
+    """The descent with a 16-lane group per query (wmax <= 8) and the one with a wavefront per query, which also writes
+    the levels: equal leaves, lists and counts, with tied scores, around whole batches of 16 roots."""
+    B, H, T = 2, 2, nb * block
+    q, k = (rnd(B, H, T, D, seed=s).mul(2).round().to(DEV).to(dtype) for s in (nb, 100 + nb))
+    perm, sums = K.forest_build(k, block, 2)
+    use = torch.randint(0, 9, (B, H, T), generator=torch.Generator().manual_seed(3)).to(DEV)
+    got = []
+    for levels in (False, True):
+        counts = torch.full((B, H, T, 2), -7, dtype=torch.int32, device=DEV)
+        leaf, leafv, cand, _ = K.forest_descend(q, sums, perm, block, wmax, bq, bq_use=use, levels=levels, counts=counts)
+        got.append((leaf, leafv, cand, counts))
+    assert all(torch.equal(a, b) for a, b in zip(*got))

@@ -100,12 +100,17 @@ __global__ __launch_bounds__(256) void level_pass_kernel(const T* __restrict__ i
 
 // The same pass with each thread holding VEC = 16 / sizeof(T) consecutive dimensions of a row, read with one
 // 16-byte load per row: TPR = D / VEC threads cover a row, so a wavefront's load instruction reads whole row
-// slices of 64 / TPR rows (64 rows apart), and each thread keeps 16 rows in flight.  Thread (slice, seg):
-// dimensions [slice VEC, slice VEC + VEC) of a segment of 64 consecutive rows, reduced by adjacent pairs with a
-// carry stack; the workgroup's NSEG = 256 / TPR segment sums are then combined pairwise in LDS, one tree level
-// per step.  Every node is (left + right) of its two children, so the nodes equal level_pass_kernel's bit for
+// slices of 64 / TPR rows (16 rows apart).  Thread (slice, seg):
+// dimensions [slice VEC, slice VEC + VEC) of a segment of 16 consecutive rows, all requested at once, reduced by
+// adjacent pairs with a carry stack; the workgroup's NSEG = 1024 / TPR segment sums are then combined pairwise in
+// LDS, one tree level per step.  Every node is (left + right) of its two children, so the nodes equal level_pass_kernel's bit for
 // bit whatever the thread layout.  Rows, level rows and the strides must keep 16-byte slices aligned.
-// (A thread holds 16 rows' loads: two batches of 8.)
+// A short sequence gives a few workgroups only and the serial chain of a segment is the time: 1024 threads with
+// segments of 16 rows cover the chunk that 256 threads with segments of 64 did, so the passes are the same.
+// (1, 6, 1024, 64) float16 over pairs of keys 23.6 -> 13.6 us, (2, 6, 4096, 64) 30.9 -> 20.6, (3, 12, 3001, 64) bfloat16 with
+// leaves of 64 19.4 -> 11.7, (4, 16, 16384, 128) 74 -> 68 us.
+constexpr int kVecThreads = 1024;
+constexpr int kVecSeg = 16;   // rows per segment
 template <typename T>
 struct VecPass {
   static constexpr int VEC = 16 / (int)sizeof(T);
@@ -125,16 +130,15 @@ __device__ __forceinline__ void store_node_vec(const LevelOut& lo, int blevel, i
 }
 
 template <typename T, int D>
-__global__ __launch_bounds__(256) void level_vec_kernel(const T* __restrict__ in, int64_t isb, int64_t ish,
+__global__ __launch_bounds__(kVecThreads) void level_vec_kernel(const T* __restrict__ in, int64_t isb, int64_t ish,
                                                         int64_t isr, int H, int n_rows, int base, int zero_first,
                                                         LevelOut lo, float* __restrict__ tot, int n_chunks) {
   constexpr int VEC = VecPass<T>::VEC;
   constexpr int TPR = D / VEC;
-  constexpr int NSEG = 256 / TPR;
-  constexpr int LOG_NSEG = NSEG == 2 ? 1 : NSEG == 4 ? 2 : NSEG == 8 ? 3 : NSEG == 16 ? 4 : NSEG == 32 ? 5 :
-                           NSEG == 64 ? 6 : 7;
-  constexpr int RB = 8;    // rows per load batch; two batches in flight
-  static_assert(TPR >= 1 && (1 << LOG_NSEG) == NSEG, "layout");
+  constexpr int NSEG = kVecThreads / TPR;
+  constexpr int LOG_NSEG = __builtin_ctz(NSEG);
+  constexpr int LSEG = __builtin_ctz(kVecSeg);
+  static_assert(TPR >= 1 && (1 << LOG_NSEG) == NSEG && (1 << LSEG) == kVecSeg, "layout");
   __shared__ __align__(16) float seg_sum[NSEG][D];
   const int sl = threadIdx.x % TPR;
   const int seg = threadIdx.x / TPR;
@@ -142,67 +146,55 @@ __global__ __launch_bounds__(256) void level_vec_kernel(const T* __restrict__ in
   const int chunk = blockIdx.x;
   const int bh = blockIdx.y;
   const int b = bh / H, h = bh % H;
-  const int64_t crow0 = (int64_t)chunk * 64 * NSEG;
-  const int64_t row0 = crow0 + seg * 64;
+  const int64_t crow0 = (int64_t)chunk * kVecSeg * NSEG;
+  const int64_t row0 = crow0 + seg * kVecSeg;
   const T* src = in + b * isb + h * ish + d0;
   const int64_t last = n_rows - 1;
 
-  float carry[7][VEC];
-  uint4 buf[2][RB];
+  float carry[LSEG + 1][VEC];
+  uint4 buf[kVecSeg];
 #pragma unroll
-  for (int i = 0; i < RB; ++i) {
+  for (int i = 0; i < kVecSeg; ++i) {
     const int64_t r = row0 + i < last ? row0 + i : last;
-    buf[0][i] = ldg16(src + r * isr);
+    buf[i] = ldg16(src + r * isr);
   }
 #pragma unroll
-  for (int bt = 0; bt < 64 / RB; ++bt) {
-    if (bt + 1 < 64 / RB) {
+  for (int i = 0; i < kVecSeg; ++i) {
+    const int64_t r = row0 + i;
+    if (r < n_rows) {
+      float x[VEC];
+      const T* e = reinterpret_cast<const T*>(&buf[i]);
 #pragma unroll
-      for (int i = 0; i < RB; ++i) {
-        const int64_t rr = row0 + (bt + 1) * RB + i;
-        const int64_t r = rr < last ? rr : last;
-        buf[(bt + 1) & 1][i] = ldg16(src + r * isr);
+      for (int v = 0; v < VEC; ++v) {
+        x[v] = (zero_first && r == 0) ? 0.0f : to_f32(e[v]);
       }
-    }
+      int lv = 0;
 #pragma unroll
-    for (int i0 = 0; i0 < RB; ++i0) {
-      const int i = bt * RB + i0;
-      const int64_t r = row0 + i;
-      if (r < n_rows) {
-        float x[VEC];
-        const T* e = reinterpret_cast<const T*>(&buf[bt & 1][i0]);
+      for (int k = 0; k < LSEG; ++k) {
+        if (((i >> k) & 1) == 0) break;
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-          x[v] = (zero_first && r == 0) ? 0.0f : to_f32(e[v]);
-        }
-        int lv = 0;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) {
-          if (((i >> k) & 1) == 0) break;
-#pragma unroll
-          for (int v = 0; v < VEC; ++v) x[v] = __fadd_rn(carry[k][v], x[v]);
-          lv = k + 1;
-          store_node_vec<VEC>(lo, base + lv, b, h, r >> lv, D, d0, x);
-        }
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) carry[lv][v] = x[v];
+        for (int v = 0; v < VEC; ++v) x[v] = __fadd_rn(carry[k][v], x[v]);
+        lv = k + 1;
+        store_node_vec<VEC>(lo, base + lv, b, h, r >> lv, D, d0, x);
       }
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) carry[lv][v] = x[v];
     }
   }
-  if (row0 + 63 < n_rows) {
+  if (row0 + kVecSeg - 1 < n_rows) {
 #pragma unroll
     for (int v = 0; v < VEC; v += 4)
       *reinterpret_cast<float4*>(&seg_sum[seg][d0 + v]) =
-          make_float4(carry[6][v], carry[6][v + 1], carry[6][v + 2], carry[6][v + 3]);
+          make_float4(carry[LSEG][v], carry[LSEG][v + 1], carry[LSEG][v + 2], carry[LSEG][v + 3]);
   }
-  // pairwise combination of the segment sums: at step k the node of binary level base + 6 + k + 1 with index p
+  // pairwise combination of the segment sums: at step k the node of binary level base + LSEG + k + 1 with index p
   // in this chunk is seg_sum[2p << k] + seg_sum[(2p + 1) << k], kept in the left child's slot
   for (int k = 0; k < LOG_NSEG; ++k) {
     __syncthreads();
     const int npairs = NSEG >> (k + 1);
-    for (int e = threadIdx.x; e < npairs * TPR; e += 256) {
+    for (int e = threadIdx.x; e < npairs * TPR; e += kVecThreads) {
       const int p = e / TPR, s2 = e % TPR;
-      const int64_t node_rows = (int64_t)64 << (k + 1);
+      const int64_t node_rows = (int64_t)kVecSeg << (k + 1);
       if (crow0 + (p + 1) * node_rows <= n_rows) {
         float* lft = &seg_sum[(2 * p) << k][s2 * VEC];
         const float* rgt = &seg_sum[(2 * p + 1) << k][s2 * VEC];
@@ -211,13 +203,13 @@ __global__ __launch_bounds__(256) void level_vec_kernel(const T* __restrict__ in
         for (int v = 0; v < VEC; ++v) x[v] = __fadd_rn(lft[v], rgt[v]);
 #pragma unroll
         for (int v = 0; v < VEC; ++v) lft[v] = x[v];
-        store_node_vec<VEC>(lo, base + 6 + k + 1, b, h, (int64_t)chunk * (NSEG >> (k + 1)) + p, D, s2 * VEC, x);
+        store_node_vec<VEC>(lo, base + LSEG + k + 1, b, h, (int64_t)chunk * (NSEG >> (k + 1)) + p, D, s2 * VEC, x);
       }
     }
   }
-  if (tot != nullptr && crow0 + 64 * NSEG <= n_rows) {
+  if (tot != nullptr && crow0 + kVecSeg * NSEG <= n_rows) {
     __syncthreads();
-    for (int e = threadIdx.x; e < D / 4; e += 256)
+    for (int e = threadIdx.x; e < D / 4; e += kVecThreads)
       *reinterpret_cast<float4*>(tot + ((int64_t)bh * n_chunks + chunk) * D + 4 * e) =
           *reinterpret_cast<const float4*>(&seg_sum[0][4 * e]);
   }
@@ -525,8 +517,8 @@ int dispatch_dt_d(int dt, int D, A&&... a) {
 
 int chunk_rows(int D) { return 64 * (256 / D); }
 
-// Rows of the pass's input a workgroup reduces: 64 rows per segment, 256 / (threads per row) segments.
-int chunk_rows_vec(int D, int elem) { return 64 * (256 / (D / (16 / elem))); }
+// Rows of the pass's input a workgroup reduces: kVecSeg rows per segment, kVecThreads / (threads per row) segments.
+int chunk_rows_vec(int D, int elem) { return kVecSeg * (kVecThreads / (D / (16 / elem))); }
 
 template <typename T, int D>
 struct LevelSumsRun {
@@ -566,8 +558,9 @@ struct LevelSumsRun {
       float* tot = more ? bufs[pass & 1] : nullptr;
       const int tot_chunks = n_rows / CH;
       dim3 grid(n_chunks, B * H);
+      const dim3 threads(vec ? kVecThreads : 256);
 #define TA_LEVEL_PASS(KER, TT, ZF)                                                                                 \
-  hipLaunchKernelGGL(KER, grid, dim3(256), 0, st, (const TT*)src, sb, sh, sr, H, n_rows, base, ZF, lo, tot, tot_chunks)
+  hipLaunchKernelGGL(KER, grid, threads, 0, st, (const TT*)src, sb, sh, sr, H, n_rows, base, ZF, lo, tot, tot_chunks)
       if (pass == 0 && logt) {
         TA_LEVEL_PASS((level_pass_kernel<T, D, true>), T, zero_sink);
       } else if (pass == 0) {

@@ -254,6 +254,16 @@ int ta_sparse_attn_bwd(const void* q, const void* k, const void* v, const void* 
                        int B, int H, int T, int Tk, int KC, int D, float scale, void* dq, float* dk, float* dv,
                        float* ws, int causal, void* stream);
 
+/* The same with the gradients' rows where the caller wants them: grad_strides holds the element strides (b, h, t) of dq,
+ * dk and dv, in that order, the last dimension contiguous, each tensor filling its memory without gaps (a permutation
+ * of a contiguous one). */
+int ta_sparse_attn_bwd_strided(const void* q, const void* k, const void* v, const void* o, const void* dout, int dtype,
+                               int64_t qsb, int64_t qsh, int64_t qst, int64_t ksb, int64_t ksh, int64_t kst,
+                               int64_t vsb, int64_t vsh, int64_t vst, int64_t osb, int64_t osh, int64_t ost,
+                               int64_t dsb, int64_t dsh, int64_t dst, const int32_t* cand, const float* lse,
+                               int B, int H, int T, int Tk, int KC, int D, float scale, void* dq, float* dk,
+                               float* dv, float* ws, int causal, const int64_t* grad_strides, void* stream);
+
 /* Bytes of the deterministic route's workspace of ta_sparse_attn_bwd (per-slot ds and p, the slots sorted by key and
  * the sort's counts); 8-byte aligned. */
 int64_t ta_sparse_attn_bwd_workspace_size(int B, int H, int T, int KC);

@@ -66,3 +66,30 @@ def test_sorted_backward_matches_float64(T, Tk, KC, D, misaligned):
     for a, b, w in zip(got, again, want):
         assert torch.equal(a, b)
         assert (a.cpu().double() - w).abs().max().item() <= 1e-5 * max(1.0, w.abs().max().item())
+
+
+@pytest.mark.parametrize('dtype,T,H,D', [(torch.float32, 130, 3, 16), (torch.float16, 77, 2, 64), (torch.bfloat16, 1, 2, 128),
+                                         (torch.float16, 33, 1, 64), (torch.float16, 50, 2, 32)])
+@pytest.mark.parametrize('case', ['views', 'offset', 'broadcast'])
+def test_strided_rows_equal_contiguous(dtype, T, H, D, case):
+    """q, k and v as views of one projection (read in place, gradients laid out alike), such views off 16-byte alignment
+    and a broadcast gradient of the output: bit for bit the contiguous tensors' results."""
+    B, KC = 2, 9
+    g = torch.Generator().manual_seed(T)
+    n = B * T * 3 * H * D
+    flat = torch.randn(n + 1, generator=g).to(dtype).to(DEV)
+    qkv = (flat[1:] if case == 'offset' else flat[:n]).view(B, T, 3 * H * D)
+    q, k, v = (t.view(B, T, H, D).transpose(1, 2) for t in qkv.split(H * D, dim=2))
+    do = torch.randn(B, T, H, D, generator=g).to(dtype).to(DEV).transpose(1, 2)
+    if case == 'broadcast':
+        do = do[:, :1, :1, :1].expand(B, H, T, D)
+    cand = torch.randint(-1, T, (B, H, T, KC), generator=g).to(DEV)
+    c = [t.contiguous() for t in (q, k, v, do)]
+    out, lse = K.sparse_attn_fwd(*c[:3], cand, 0.125)
+    want = K.sparse_attn_bwd(*c[:3], cand, 0.125, out, lse, c[3], deterministic=True)
+    got = K.sparse_attn_bwd(q, k, v, cand, 0.125, out, lse, do, deterministic=True)
+    assert all(torch.equal(a, b) and a.dtype == b.dtype for a, b in zip(got, want))
+    # atomic adds: float32 sums of up to T KC terms in any order, rounded to the type
+    tol = {torch.float32: 1e-5, torch.float16: 2e-3, torch.bfloat16: 1.6e-2}[dtype]
+    for a, b in zip(K.sparse_attn_bwd(q, k, v, cand, 0.125, out, lse, do, deterministic=False), want):
+        assert (a.float() - b.float()).abs().max().item() <= tol * max(1.0, b.float().abs().max().item())

@@ -32,8 +32,8 @@ struct BwdParams {
   int64_t qsb, qsh, qst, ksb, ksh, kst, vsb, vsh, vst, osb, osh, ost, dsb, dsh, dst;
   const int32_t* cand;   // (B,H,T,KC) contiguous
   const float* lse;      // (B,H,T) contiguous
-  void* dq;              // (B,H,T,D) contiguous, input dtype
-  float *dk, *dv;        // (B,H,Tk,D) contiguous float32: accumulated into (atomics) or written (workspace)
+  void* dq;              // (B,H,T,D) rows, input dtype
+  float *dk, *dv;        // (B,H,Tk,D) rows, float32: accumulated into (atomics) or written (workspace)
   float2* dsp;           // (B,H,T,KC) per-slot (ds, p), written where the slot is valid (the sorted route), or null
   uint2* ent;            // (B,H,T*KC) sorted entries: slot index, query << kLowBits | key within its bucket
   int32_t* cnt;          // per (b,h): [bucket][chunk] counts, then starts; one more word: the number of entries
@@ -42,6 +42,7 @@ struct BwdParams {
   int rows_al;           // q, o and do rows, dq, dk and dv are 16-byte aligned
   int CQ, NC;            // queries per chunk, chunks
   int wlog, NB;          // log2 of a bucket's keys, buckets
+  int64_t gq[3], gk[3], gv[3];   // strides (b, h, row) of dq, dk, dv
 };
 
 constexpr int kBwdMaxD = 256;
@@ -175,8 +176,8 @@ __global__ __launch_bounds__(kWave * kBwdWaves) void bwd_query_kernel(BwdParams 
         if (p.dsp != nullptr) {
           if (d0 == 0) p.dsp[row * p.KC + s_slot[wv][i]] = make_float2(ds, pw);
         } else if (in) {
-          float* dkr = p.dk + ((int64_t)bh * p.Tk + jr) * D + d0;
-          float* dvr = p.dv + ((int64_t)bh * p.Tk + jr) * D + d0;
+          float* dkr = p.dk + b * p.gk[0] + h * p.gk[1] + jr * p.gk[2] + d0;
+          float* dvr = p.dv + b * p.gv[0] + h * p.gv[1] + jr * p.gv[2] + d0;
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             atomicAdd(dkr + e, p.scale * ds * qf[e]);
@@ -189,7 +190,7 @@ __global__ __launch_bounds__(kWave * kBwdWaves) void bwd_query_kernel(BwdParams 
   }
 #pragma unroll
   for (int e = 0; e < 8; ++e) dq[e] = p.scale * across_groups<L>(dq[e]);
-  if (g == 0 && in) store8(reinterpret_cast<T*>(p.dq) + row * D + d0, al, dq);
+  if (g == 0 && in) store8(reinterpret_cast<T*>(p.dq) + b * p.gq[0] + h * p.gq[1] + t * p.gq[2] + d0, al, dq);
 }
 
 // ---------------------------------------------------------------------------------- sorting the slots by key
@@ -404,8 +405,8 @@ __global__ __launch_bounds__(kWave * kKeyWaves, 4) void bwd_keys_kernel(BwdParam
   const int dl = in ? d0 : 0;   // lanes past the row read its first slice and write nothing
   const T* qb = reinterpret_cast<const T*>(p.q) + b * p.qsb + h * p.qsh + dl;
   const T* db = reinterpret_cast<const T*>(p.dout) + b * p.dsb + h * p.dsh + dl;
-  float* dkb = p.dk + ((int64_t)bh * p.Tk + j0) * D;
-  float* dvb = p.dv + ((int64_t)bh * p.Tk + j0) * D;
+  float* dkb = p.dk + b * p.gk[0] + h * p.gk[1] + j0 * p.gk[2];
+  float* dvb = p.dv + b * p.gv[0] + h * p.gv[1] + j0 * p.gv[2];
   const uint64_t below = (1ull << lane) - 1;
   constexpr uint32_t kLow = (1u << kLowBits) - 1;
   uint16_t* list = s_list[wv];
@@ -436,8 +437,8 @@ __global__ __launch_bounds__(kWave * kKeyWaves, 4) void bwd_keys_kernel(BwdParam
       if (key >= nk || len > kHeavy || (len == 0 && !fresh)) continue;
       key_part<T, L, VEC, 2>(p, qb, db, dsp, s_e, list, len, g, dk, dv);
       if (g == 0 && in) {
-        float* dkr = dkb + (int64_t)key * D + d0;
-        float* dvr = dvb + (int64_t)key * D + d0;
+        float* dkr = dkb + key * p.gk[2] + d0;
+        float* dvr = dvb + key * p.gv[2] + d0;
         if (!fresh) {
 #pragma unroll
           for (int x = 0; x < 8; ++x) {
@@ -469,7 +470,7 @@ __global__ __launch_bounds__(kWave * kKeyWaves, 4) void bwd_keys_kernel(BwdParam
         float sum = 0.0f;
 #pragma unroll
         for (int u = 0; u < kKeyWaves; ++u) sum += s_part[u][which][dd];
-        float* r = (which ? dvb : dkb) + (int64_t)key * D + dd;
+        float* r = (which ? dvb + key * p.gv[2] : dkb + key * p.gk[2]) + dd;
         *r = fresh ? sum : *r + sum;
       }
       __syncthreads();
@@ -533,12 +534,12 @@ static void launch_bwd_d(const BwdParams& p, bool sorted, hipStream_t st) {
 
 using namespace ta;
 
-extern "C" int ta_sparse_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout,
+static int sparse_attn_bwd_impl(const void* q, const void* k, const void* v, const void* o, const void* dout,
                                   int dtype, int64_t qsb, int64_t qsh, int64_t qst, int64_t ksb, int64_t ksh,
                                   int64_t kst, int64_t vsb, int64_t vsh, int64_t vst, int64_t osb, int64_t osh,
                                   int64_t ost, int64_t dsb, int64_t dsh, int64_t dst, const int32_t* cand,
                                   const float* lse, int B, int H, int T, int Tk, int KC, int D, float scale,
-                                  void* dq, float* dk, float* dv, float* ws, int causal, void* stream) {
+                                  void* dq, float* dk, float* dv, float* ws, const int64_t* gs, void* stream) {
   if (B < 0 || H < 0 || T < 0 || Tk <= 0 || KC < 0 || D <= 0 || D > kBwdMaxD || D % 8) {
     set_error("ta_sparse_attn_bwd: bad sizes (D a multiple of 8, at most 256)");
     return TA_ERR_ARG;
@@ -562,9 +563,10 @@ extern "C" int ta_sparse_attn_bwd(const void* q, const void* k, const void* v, c
   // rows of q, o, dout, dq, dk and dv are moved 8 elements at a time where all are aligned, else one by one
   const int al = !(((uintptr_t)q | (uintptr_t)o | (uintptr_t)dout | (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) % 16 || (qsb * es) % 16 || (qsh * es) % 16 ||
                    (qst * es) % 16 || (osb * es) % 16 || (osh * es) % 16 || (ost * es) % 16 || (dsb * es) % 16 ||
-                   (dsh * es) % 16 || (dst * es) % 16);
+                   (dsh * es) % 16 || (dst * es) % 16 || ((gs[0] | gs[1] | gs[2]) * es) % 16 ||
+                   ((gs[3] | gs[4] | gs[5] | gs[6] | gs[7] | gs[8]) * 4) % 16);
   BwdParams p{q, k, v, o, dout, qsb, qsh, qst, ksb, ksh, kst, vsb, vsh, vst, osb, osh, ost, dsb, dsh, dst,
-              cand, lse, dq, dk, dv, nullptr, nullptr, nullptr, B, H, T, Tk, KC, D, scale, al, 0, 0, 0, 0};
+              cand, lse, dq, dk, dv, nullptr, nullptr, nullptr, B, H, T, Tk, KC, D, scale, al, 0, 0, 0, 0, {gs[0], gs[1], gs[2]}, {gs[3], gs[4], gs[5]}, {gs[6], gs[7], gs[8]}};
   hipStream_t st = (hipStream_t)stream;
   bool sorted = ws != nullptr && KC > 0;
   if (sorted) {
@@ -588,6 +590,33 @@ extern "C" int ta_sparse_attn_bwd(const void* q, const void* k, const void* v, c
     default: launch_bwd_d<bf16_t>(p, sorted, st); break;
   }
   return check_launch("ta_sparse_attn_bwd");
+}
+
+extern "C" int ta_sparse_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout,
+                                  int dtype, int64_t qsb, int64_t qsh, int64_t qst, int64_t ksb, int64_t ksh,
+                                  int64_t kst, int64_t vsb, int64_t vsh, int64_t vst, int64_t osb, int64_t osh,
+                                  int64_t ost, int64_t dsb, int64_t dsh, int64_t dst, const int32_t* cand,
+                                  const float* lse, int B, int H, int T, int Tk, int KC, int D, float scale,
+                                  void* dq, float* dk, float* dv, float* ws, int, void* stream) {
+  const int64_t hq = (int64_t)T * D, hk = (int64_t)Tk * D;
+  const int64_t gs[9] = {H * hq, hq, D, H * hk, hk, D, H * hk, hk, D};
+  return sparse_attn_bwd_impl(q, k, v, o, dout, dtype, qsb, qsh, qst, ksb, ksh, kst, vsb, vsh, vst, osb, osh, ost, dsb,
+                              dsh, dst, cand, lse, B, H, T, Tk, KC, D, scale, dq, dk, dv, ws, gs, stream);
+}
+
+extern "C" int ta_sparse_attn_bwd_strided(const void* q, const void* k, const void* v, const void* o, const void* dout,
+                                          int dtype, int64_t qsb, int64_t qsh, int64_t qst, int64_t ksb, int64_t ksh,
+                                          int64_t kst, int64_t vsb, int64_t vsh, int64_t vst, int64_t osb,
+                                          int64_t osh, int64_t ost, int64_t dsb, int64_t dsh, int64_t dst,
+                                          const int32_t* cand, const float* lse, int B, int H, int T, int Tk, int KC,
+                                          int D, float scale, void* dq, float* dk, float* dv, float* ws, int,
+                                          const int64_t* grad_strides, void* stream) {
+  if (grad_strides == nullptr) {
+    set_error("ta_sparse_attn_bwd_strided: no strides of the gradients");
+    return TA_ERR_ARG;
+  }
+  return sparse_attn_bwd_impl(q, k, v, o, dout, dtype, qsb, qsh, qst, ksb, ksh, kst, vsb, vsh, vst, osb, osh, ost, dsb,
+                              dsh, dst, cand, lse, B, H, T, Tk, KC, D, scale, dq, dk, dv, ws, grad_strides, stream);
 }
 
 // Workspace of the sorted dk / dv route of ta_sparse_attn_bwd: per-slot (ds, p), the sorted entries, and the counts of

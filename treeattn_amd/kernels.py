@@ -650,6 +650,22 @@ def dkdv_scan_ints(B, H, T, Tk, KC, D, causal):
     return B * H * rows * KC
 
 
+def _read_rows(t):
+    """t, or its contiguous copy where the backward's 16-byte reads do not fit its rows."""
+    es = t.element_size()
+    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s * es % 16 == 0 for s in t.stride()[:-1])
+    return t if ok else t.contiguous()
+
+
+def _grad_rows(t, alloc, dtype):
+    """An (b,H,T,D) gradient with its rows in t's order: heads inside positions where t is a projection's view, so that
+    the gradient of the projection takes it without a copy (two copies of 6.5 us per tensor at (2, 6, 4096, 64))."""
+    b, H, T, D = t.shape
+    if H > 1 and T > 1 and t.stride(1) < t.stride(2):
+        return alloc(b, T, H, D, device=t.device, dtype=dtype).transpose(1, 2)
+    return alloc(b, H, T, D, device=t.device, dtype=dtype)
+
+
 def sparse_attn_bwd(q, k, v, cand, scale, out, lse, dout, deterministic=None, causal=False):
     """Gradients of sparse_attn_fwd: (dq in q's dtype, dk, dv in k's / v's dtype).  dk and dv are summed in
     float32: deterministic, in a fixed order (the slots sorted by key, queries then slots ascending) through a
@@ -659,13 +675,13 @@ def sparse_attn_bwd(q, k, v, cand, scale, out, lse, dout, deterministic=None, ca
     L.require_gpu(q, k, v, cand, out, lse, dout)
     if not (q.dtype == k.dtype == v.dtype == out.dtype):
         raise TypeError('q, k, v and out must share a dtype')
-    q, k, v, out, dout = [t.contiguous() for t in (q, k, v, out, dout.to(q.dtype))]
+    q, k, v, out, dout = [_read_rows(t) for t in (q, k, v, out, dout.to(q.dtype))]
     b, H, T, D = q.shape
     Tk = k.shape[2]
     KC = cand.shape[-1]
     cc = cand.to(torch.int32).contiguous()
     ls = lse.float().contiguous()
-    dq = torch.empty_like(q)
+    dq = _grad_rows(q, torch.empty, q.dtype)
     ws = None
     if deterministic is None:
         deterministic = dkdv_scan_ints(b, H, T, Tk, KC, D, causal and T == Tk) <= DKDV_SCAN_LIMIT
@@ -673,12 +689,13 @@ def sparse_attn_bwd(q, k, v, cand, scale, out, lse, dout, deterministic=None, ca
         nbytes = L.lib().ta_sparse_attn_bwd_workspace_size(b, H, T, KC)
         ws = torch.empty(max(1, nbytes // 4), device=q.device, dtype=torch.float32)
     alloc = torch.empty if ws is not None else torch.zeros   # written whole, or accumulated into
-    dk = alloc(k.shape, device=q.device, dtype=torch.float32)
-    dv = alloc(v.shape, device=q.device, dtype=torch.float32)
-    L.call('ta_sparse_attn_bwd', L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(out), L.ptr(dout), L.dtype_code(q),
+    dk = _grad_rows(k, alloc, torch.float32)
+    dv = _grad_rows(v, alloc, torch.float32)
+    strides = L.i64_array([s for t in (dq, dk, dv) for s in t.stride()[:3]])
+    L.call('ta_sparse_attn_bwd_strided', L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(out), L.ptr(dout), L.dtype_code(q),
            *L.rows3(q), *L.rows3(k), *L.rows3(v), *L.rows3(out), *L.rows3(dout), L.ptr(cc), L.ptr(ls), b, H, T, Tk,
            KC, D, float(scale), L.ptr(dq), L.ptr(dk), L.ptr(dv), L.ptr(ws), 1 if (causal and T == Tk) else 0,
-           L.stream())
+           strides, L.stream())
     return dq, dk.to(k.dtype), dv.to(v.dtype)
 
 

@@ -1,7 +1,7 @@
 // Sparse softmax attention on gfx950 over the keys a query selected, and the decode-cache append.
 //
 // One wavefront per (query, split).  The query's keys are enumerated as a flat list (selected leaf blocks,
-// the own partial leaf block, the static keys not already covered); a
+// the own partial leaf block, the static keys not already covered -- or an explicit candidate list); a
 // chunk of the list maps one key to each lane (two lanes per key when D = 128).  Each lane reads its key's
 // K and V rows (a leaf block is a run of consecutive rows, so a chunk reads contiguous memory), keeps a
 // running max/sum (online softmax, float32) and its own weighted V accumulator; the wavefront reduces
@@ -26,7 +26,7 @@ namespace ta {
 
 
 // PIPE: the copy-free chunk loop of attn_query, for several workgroups per query (p.gsplit > 1).
-template <typename T, int D, bool SPLIT, bool PIPE = false>
+template <typename T, int D, bool SPLIT, bool CAND, bool PIPE = false>
 __global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
   extern __shared__ float smem_f[];
   const int w = wave_id();
@@ -43,9 +43,16 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
   const int64_t qi = (int64_t)bh * p.Nq + n;
   const T* qrow = reinterpret_cast<const T*>(p.q) + b * p.qsb + h * p.qsh + n * p.qsn;
   T* orow = reinterpret_cast<T*>(p.out) + b * p.osb + h * p.osh + n * p.osn;
-  const int t = p.tq[b * p.tq_sb + n];
-  const int nt = p.n_tree ? p.n_tree[qi] : p.wl;
-  attn_query<T, D, SPLIT, PIPE>(p, n, g, b, h, qi, qrow, t, p.ids + qi * p.wl, p.vld + qi * p.wl, -1, nt, orow, smem_f);
+  int t = 0, nt = 0;
+  const int32_t* idr = nullptr;
+  const uint8_t* vr = nullptr;
+  if constexpr (!CAND) {
+    t = p.tq[b * p.tq_sb + n];
+    idr = p.ids + qi * p.wl;
+    vr = p.vld + qi * p.wl;
+    nt = p.n_tree ? p.n_tree[qi] : p.wl;
+  }
+  attn_query<T, D, SPLIT, CAND, PIPE>(p, n, g, b, h, qi, qrow, t, idr, vr, -1, nt, orow, smem_f);
 }
 
 // ----------------------------------------------------------------------------------------- decode attend
@@ -116,7 +123,7 @@ __global__ __launch_bounds__(kWavesPerBlock * kWave) void seg_attend_kernel(Attn
   const int nt = p.n_tree ? p.n_tree[bh] : p.wl;
   T* orow = reinterpret_cast<T*>(p.out) + b * p.osb + h * p.osh;
   TA_DMARK(14);
-  attn_query<T, D, true>(p, 0, 0, b, h, bh, qrow, t, kid, nullptr, nkw, nt, orow, att, kpg, s_pre);
+  attn_query<T, D, true, false>(p, 0, 0, b, h, bh, qrow, t, kid, nullptr, nkw, nt, orow, att, kpg, s_pre);
   TA_DMARK(15);
   const int64_t obase = (int64_t)bh * p.wl;   // kid and ksc are not written by the attention
   for (int r = tid; r < p.wl; r += NT) {
@@ -152,160 +159,6 @@ __global__ __launch_bounds__(256) void kv_append_kernel(AppendIn ap, int H, int 
                 leaf_log2, arity_log2, stk, [&](int j) { return lv.ptr[j] + b * lv.sb[j] + h * lv.sh[j]; });
 }
 
-// ----------------------------------------------------------------------------------------- candidate lists
-// Attention of many queries over explicit candidate lists (the modules' default selection: leaves of two keys, so
-// a list has 30 to 90 slots of which about 20 hold a key).  One wavefront per query.  The list is read 64 slots
-// at a time, its valid rows are packed into LDS by ballots, and only those are attended: NL load instructions of
-// K and as many of V per batch, all requested at once (32 keys of 8 dims a lane in 16 bits: a typical list is one
-// batch).  The row groups' accumulators are summed by halving: at each step a lane sends the half of its
-// dimensions that its partner keeps, 7 exchanges for 8 dims over 8 groups where summing every dim takes 24, and
-// all lanes store.  What bounds it is the instructions of a wavefront (4 cycles each), not the rows it reads.
-// (2, 6, 4096, 64) float16 with lists of 52: 110.7 -> 46.2 us; (1, 6, 4096, 64) with lists of 83: 79.2 -> 42.5; (8, 6, 512,
-// 64) float32: 61.5 -> 25.2; (1, 6, 1024, 64): 17.1 -> 9.5 (before: every slot fetched, the empty ones too).
-constexpr int kListCap = 256;   // slots packed at a time (longer lists: in several passes, the softmax running on)
-
-template <typename T, int D>
-__global__ __launch_bounds__(kWavesPerBlock * kWave) void attn_list_kernel(AttnParams p) {
-  constexpr int EPL = Raw16<T>::EPL;
-  constexpr int LPR = D / EPL;      // lanes per key row
-  constexpr int RPI = kWave / LPR;  // key rows per load instruction
-  constexpr int NL = RPI >= 16 ? 2 : RPI == 8 ? 4 : 8;
-  constexpr int KPC = NL * RPI;
-  __shared__ int32_t s_rows[kWavesPerBlock][kListCap];
-  const int lane = lane_id(), w = wave_id();
-  const int n = blockIdx.x * kWavesPerBlock + w;
-  if (n >= p.Nq) return;   // no workgroup barrier below
-  const int bh = blockIdx.y;
-  const int b = bh / p.H, h = bh % p.H;
-  const int64_t qi = (int64_t)bh * p.Nq + n;
-  const int rg = lane / LPR;
-  const int ds = (lane % LPR) * EPL;
-  int32_t* rows = s_rows[w];
-  const int32_t* crow = p.cand + qi * p.KC;
-  const int32_t* ptrow = p.ptab ? p.ptab + b * p.pt_sb + h * p.pt_sh : nullptr;
-  const int rpp = ptrow ? (int)(p.kps / p.kst) : 0;   // rows from one page to the next
-  float qv[EPL];
-  load_row<T, EPL>(reinterpret_cast<const T*>(p.q) + b * p.qsb + h * p.qsh + n * p.qsn + ds, qv);
-  const char* kb = reinterpret_cast<const char*>(reinterpret_cast<const T*>(p.k) + b * p.ksb + h * p.ksh + ds);
-  const char* vb = reinterpret_cast<const char*>(reinterpret_cast<const T*>(p.v) + b * p.vsb + h * p.vsh + ds);
-  const int64_t kst_b = p.kst * (int64_t)sizeof(T), vst_b = p.vst * (int64_t)sizeof(T);
-
-  float m = kNegBig, l = 0.0f;   // of this lane's row group, the same in its LPR lanes
-  float acc[EPL];
-#pragma unroll
-  for (int d = 0; d < EPL; ++d) acc[d] = 0.0f;
-
-  for (int base = 0; base < p.KC; base += kListCap) {
-    int pos[kListCap / kWave];
-#pragma unroll
-    for (int j = 0; j < kListCap / kWave; ++j) {
-      const int c = base + j * kWave + lane;
-      pos[j] = c < p.KC ? crow[c] : -1;
-    }
-    int cnt = 0;
-#pragma unroll
-    for (int j = 0; j < kListCap / kWave; ++j) {
-      if (base + j * kWave < p.KC) {
-        int row = pos[j] < p.Tk ? pos[j] : -1;
-        if (ptrow != nullptr && row >= 0) {
-          const int pg = ptrow[row >> p.leaf_log2];
-          row = (pg >= 0 && pg < p.npages) ? pg * rpp + (row & ((1 << p.leaf_log2) - 1)) : -1;
-        }
-        const uint64_t bal = __ballot(row >= 0);
-        if (row >= 0) rows[cnt + __popcll(bal & ((1ull << lane) - 1))] = row;
-        cnt += __popcll(bal);
-      }
-    }
-    wave_sync();
-    for (int k0 = 0; k0 < cnt; k0 += KPC) {
-      uint4 kr[NL], vr[NL];
-      bool ok[NL];
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        const int key = k0 + i * RPI + rg;
-        ok[i] = key < cnt;
-        const int64_t r = rows[ok[i] ? key : k0];
-        kr[i] = ldg16(kb + r * kst_b);
-        vr[i] = ldg16(vb + r * vst_b);
-      }
-      float sc[NL];
-      float mn = m;
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        float kv[EPL];
-        Raw16<T>::cvt(kr[i], kv);
-        float d0 = 0.0f;
-#pragma unroll
-        for (int d = 0; d < EPL; ++d) d0 = fmaf(qv[d], kv[d], d0);
-        sc[i] = d0;
-      }
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        const float d0 = group_sum<LPR>(sc[i]) * p.scale;
-        sc[i] = ok[i] ? d0 : kNegBig;
-        mn = fmaxf(mn, sc[i]);
-      }
-      const float alpha = __expf(m - mn);
-#pragma unroll
-      for (int d = 0; d < EPL; ++d) acc[d] *= alpha;
-      l *= alpha;
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        // a slot past the list adds nothing, whatever the row read in its place holds
-        const float pw = ok[i] ? __expf(sc[i] - mn) : 0.0f;
-        if (!ok[i]) vr[i] = make_uint4(0, 0, 0, 0);
-        l += pw;
-        float vv[EPL];
-        Raw16<T>::cvt(vr[i], vv);
-#pragma unroll
-        for (int d = 0; d < EPL; ++d) acc[d] = fmaf(pw, vv[d], acc[d]);
-      }
-      m = mn;
-    }
-    wave_sync();   // the list is read before the next pass overwrites it
-  }
-
-  // the row groups to one maximum, their sums, and the accumulators' sum by halving
-  float M = m;
-#pragma unroll
-  for (int o = LPR; o < kWave; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, kWave));
-  const float f = __expf(m - M);
-  float L = l * f;
-#pragma unroll
-  for (int o = LPR; o < kWave; o <<= 1) L += __shfl_xor(L, o, kWave);
-#pragma unroll
-  for (int d = 0; d < EPL; ++d) acc[d] *= f;
-  int e0 = 0;          // first dimension of the slice this lane ends with
-  int keep = EPL;      // how many (known at compile time after unrolling)
-  bool writes = true;  // groups past EPL hold the same dimension: one of them stores
-#pragma unroll
-  for (int o = kWave / 2; o >= LPR; o >>= 1) {
-    const bool up = (lane & o) != 0;
-    if (keep > 1) {
-      keep >>= 1;
-#pragma unroll
-      for (int d = 0; d < EPL / 2; ++d)
-        if (d < keep) {
-          const float send = up ? acc[d] : acc[d + keep];
-          const float own = up ? acc[d + keep] : acc[d];
-          acc[d] = own + __shfl_xor(send, o, kWave);
-        }
-      e0 += up ? keep : 0;
-    } else {
-      acc[0] += __shfl_xor(acc[0], o, kWave);
-      writes = writes && !up;
-    }
-  }
-  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-  T* orow = reinterpret_cast<T*>(p.out) + b * p.osb + h * p.osh + n * p.osn + ds + e0;
-  if (writes) {
-#pragma unroll
-    for (int d = 0; d < EPL; ++d)
-      if (d < keep) orow[d] = from_f32<T>(acc[d] * inv);
-  }
-  if (lane == 0 && p.lse) p.lse[qi] = L > 0.0f ? M + __logf(L) : kNegBig;
-}
-
 // ----------------------------------------------------------------------------------------- host side
 namespace {
 
@@ -324,19 +177,24 @@ bool kv_aligned(const void* p, int dt, int D, std::initializer_list<int64_t> str
 
 template <typename T, int D>
 int launch_attn(const AttnParams& p, int B, bool split, hipStream_t st) {
-  const int wl_pad = attn_list_cap(p.wl, p.nb_S);
+  const int wl_pad = p.cand ? 0 : attn_list_cap(p.wl, p.nb_S);
   size_t lds = (size_t)kWavesPerBlock * attn_wave_ints(wl_pad) * sizeof(float);
   const dim3 blk(kWavesPerBlock * kWave);
   if (split) {
     lds += (size_t)kWavesPerBlock * (D + 2) * sizeof(float);
     dim3 grid((unsigned)((int64_t)p.Nq * p.gsplit), B * p.H);
-    if (p.gsplit > 1) hipLaunchKernelGGL((attn_kernel<T, D, true, true>), grid, blk, lds, st, p);
-    else hipLaunchKernelGGL((attn_kernel<T, D, true>), grid, blk, lds, st, p);
+    if (p.gsplit > 1) {
+      if (p.cand) hipLaunchKernelGGL((attn_kernel<T, D, true, true, true>), grid, blk, lds, st, p);
+      else hipLaunchKernelGGL((attn_kernel<T, D, true, false, true>), grid, blk, lds, st, p);
+    } else {
+      if (p.cand) hipLaunchKernelGGL((attn_kernel<T, D, true, true>), grid, blk, lds, st, p);
+      else hipLaunchKernelGGL((attn_kernel<T, D, true, false>), grid, blk, lds, st, p);
+    }
     return check_launch("attn_kernel");
   }
   dim3 grid((unsigned)((p.Nq + kWavesPerBlock - 1) / kWavesPerBlock), B * p.H);
-  if (p.cand) hipLaunchKernelGGL((attn_list_kernel<T, D>), grid, blk, 0, st, p);
-  else hipLaunchKernelGGL((attn_kernel<T, D, false>), grid, blk, lds, st, p);
+  if (p.cand) hipLaunchKernelGGL((attn_kernel<T, D, false, true>), grid, blk, lds, st, p);
+  else hipLaunchKernelGGL((attn_kernel<T, D, false, false>), grid, blk, lds, st, p);
   return check_launch("attn_kernel");
 }
 

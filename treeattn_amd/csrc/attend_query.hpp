@@ -58,7 +58,7 @@ template <> struct Raw16<f16_t> {
 // Paged caches: pre_leaf_pg (LDS, may be null) holds the pages of the leaf blocks idr lists and pre_static_pg
 // (LDS, may be null) the page of static slot i's block (slot 0: position 0, slot i >= 1: position t - i + 1),
 // read earlier by the caller; when null they are looked up in the page table here.
-template <typename T, int D, bool SPLIT, bool PIPE = false>
+template <typename T, int D, bool SPLIT, bool CAND, bool PIPE = false>
 __device__ __forceinline__ void attn_query(const AttnParams& p, int n, int g, int b, int h, int64_t qi, const T* qrow,
                                            int t, const int32_t* idr, const uint8_t* vr, int nv_given, int nt,
                                            T* orow_base, float* smem_f, const int32_t* pre_leaf_pg = nullptr,
@@ -73,7 +73,7 @@ __device__ __forceinline__ void attn_query(const AttnParams& p, int n, int g, in
   (void)n;
   (void)b;
   (void)h;
-  const int wl_pad = attn_list_cap(p.wl, p.nb_S);
+  const int wl_pad = p.cand ? 0 : attn_list_cap(p.wl, p.nb_S);
   // per wavefront: used leaf ids [wl_pad], their pages [wl_pad], static keys [32] and their pages [32]
   int32_t* s_ids = reinterpret_cast<int32_t*>(smem_f + w * attn_wave_ints(wl_pad));
   int32_t* s_row0 = s_ids + wl_pad;
@@ -95,70 +95,74 @@ __device__ __forceinline__ void attn_query(const AttnParams& p, int n, int g, in
   // key list of this query
   int N, nused = 0, lb = 0, nloc = 0, next = 0, own0 = -1;
   const int leaf = 1 << p.leaf_log2;
-  if (t >= p.Tk) t = -1;  // out of range: attend nothing
-  int nv = nv_given;
-  if (nv < 0) {
-    nv = 0;
-    for (int i0 = 0; i0 < p.wl; i0 += kWave) {
-      const int i = i0 + lane;
-      const bool v = i < p.wl && vr[i] != 0;
-      nv += __popcll(__ballot(v));
+  if constexpr (CAND) {
+    N = p.KC;
+  } else {
+    if (t >= p.Tk) t = -1;  // out of range: attend nothing
+    int nv = nv_given;
+    if (nv < 0) {
+      nv = 0;
+      for (int i0 = 0; i0 < p.wl; i0 += kWave) {
+        const int i = i0 + lane;
+        const bool v = i < p.wl && vr[i] != 0;
+        nv += __popcll(__ballot(v));
+      }
     }
-  }
-  nused = t < 0 ? 0 : (nv < nt ? nv : (nt > 0 ? nt : 0));
-  for (int i = lane; i < nused; i += kWave) {
-    const int id = idr[i];
-    s_ids[i] = id;
-    s_row0[i] = (pre_leaf_pg != nullptr && ptrow != nullptr) ? row0_pg(pre_leaf_pg[i]) : row0_of(id);
-  }
-  lb = t < 0 ? 0 : (t >> p.leaf_log2) << p.leaf_log2;
-  nloc = t < 0 ? 0 : t - lb + 1;
-  wave_sync();
-  if (p.nb_S > 0 && t >= 0) {
-    // neighbour leaves: a matched slot joins when its block is complete before the own block, is not one of the
-    // tree leaves and no earlier matched slot holds the same leaf (the reference's first-copy dedupe of
-    // [tree | neighbour | static] positions, fastseg.py:376-381, as a set of leaf blocks)
-    const bool in = lane < p.nb_S;
-    const int id = in ? p.nb_id[qi * p.nb_S + lane] : -1;
-    const bool cand = in && p.nb_ok[qi * p.nb_S + lane] != 0 && id >= 0;
-    bool keepn = cand && id < (lb >> p.leaf_log2);
-    for (int i = 0; i < nused; ++i)
-      if (s_ids[i] == id) keepn = false;
-    const uint64_t cm = __ballot(cand);
-    for (int s2 = 0; s2 < p.nb_S; ++s2) {
-      const int o = __shfl(id, s2, kWave);
-      if (((cm >> s2) & 1) && s2 < lane && o == id) keepn = false;
+    nused = t < 0 ? 0 : (nv < nt ? nv : (nt > 0 ? nt : 0));
+    for (int i = lane; i < nused; i += kWave) {
+      const int id = idr[i];
+      s_ids[i] = id;
+      s_row0[i] = (pre_leaf_pg != nullptr && ptrow != nullptr) ? row0_pg(pre_leaf_pg[i]) : row0_of(id);
     }
-    const uint64_t km = __ballot(keepn);
-    if (keepn) {
-      const int slot = nused + __popcll(km & ((1ull << lane) - 1));
-      s_ids[slot] = id;
-      s_row0[slot] = row0_of(id);
-    }
-    nused += __popcll(km);
+    lb = t < 0 ? 0 : (t >> p.leaf_log2) << p.leaf_log2;
+    nloc = t < 0 ? 0 : t - lb + 1;
     wave_sync();
+    if (p.nb_S > 0 && t >= 0) {
+      // neighbour leaves: a matched slot joins when its block is complete before the own block, is not one of the
+      // tree leaves and no earlier matched slot holds the same leaf (the reference's first-copy dedupe of
+      // [tree | neighbour | static] positions, fastseg.py:376-381, as a set of leaf blocks)
+      const bool in = lane < p.nb_S;
+      const int id = in ? p.nb_id[qi * p.nb_S + lane] : -1;
+      const bool cand = in && p.nb_ok[qi * p.nb_S + lane] != 0 && id >= 0;
+      bool keepn = cand && id < (lb >> p.leaf_log2);
+      for (int i = 0; i < nused; ++i)
+        if (s_ids[i] == id) keepn = false;
+      const uint64_t cm = __ballot(cand);
+      for (int s2 = 0; s2 < p.nb_S; ++s2) {
+        const int o = __shfl(id, s2, kWave);
+        if (((cm >> s2) & 1) && s2 < lane && o == id) keepn = false;
+      }
+      const uint64_t km = __ballot(keepn);
+      if (keepn) {
+        const int slot = nused + __popcll(km & ((1ull << lane) - 1));
+        s_ids[slot] = id;
+        s_row0[slot] = row0_of(id);
+      }
+      nused += __popcll(km);
+      wave_sync();
+    }
+    // static keys [0, t, t-1, ..., t-Lw+1]: keep those >= 0, outside the own block, whose leaf block is
+    // not used, and not a repeat of the sink
+    int pe = -1;
+    if (lane <= p.Lw && t >= 0) pe = lane == 0 ? 0 : t - (lane - 1);
+    bool keep = pe >= 0 && pe < lb && !(lane > 0 && pe == 0);
+    if (keep) {
+      const int lf = pe >> p.leaf_log2;
+      for (int i = 0; i < nused; ++i)
+        if (s_ids[i] == lf) keep = false;
+    }
+    const uint64_t bal = __ballot(keep);
+    if (keep) {
+      const int slot = __popcll(bal & ((1ull << lane) - 1));
+      const int r0 = (pre_static_pg != nullptr && ptrow != nullptr) ? row0_pg(pre_static_pg[lane])
+                                                                    : row0_of(pe >> p.leaf_log2);
+      s_ext[slot] = r0 < 0 ? -1 : r0 + (pe & (leaf - 1));
+    }
+    next = __popcll(bal);
+    N = nused * leaf + nloc + next;
+    own0 = t < 0 ? -1 : ((pre_static_pg != nullptr && ptrow != nullptr) ? row0_pg(pre_static_pg[1])
+                                                                        : row0_of(t >> p.leaf_log2));
   }
-  // static keys [0, t, t-1, ..., t-Lw+1]: keep those >= 0, outside the own block, whose leaf block is
-  // not used, and not a repeat of the sink
-  int pe = -1;
-  if (lane <= p.Lw && t >= 0) pe = lane == 0 ? 0 : t - (lane - 1);
-  bool keep = pe >= 0 && pe < lb && !(lane > 0 && pe == 0);
-  if (keep) {
-    const int lf = pe >> p.leaf_log2;
-    for (int i = 0; i < nused; ++i)
-      if (s_ids[i] == lf) keep = false;
-  }
-  const uint64_t bal = __ballot(keep);
-  if (keep) {
-    const int slot = __popcll(bal & ((1ull << lane) - 1));
-    const int r0 = (pre_static_pg != nullptr && ptrow != nullptr) ? row0_pg(pre_static_pg[lane])
-                                                                  : row0_of(pe >> p.leaf_log2);
-    s_ext[slot] = r0 < 0 ? -1 : r0 + (pe & (leaf - 1));
-  }
-  next = __popcll(bal);
-  N = nused * leaf + nloc + next;
-  own0 = t < 0 ? -1 : ((pre_static_pg != nullptr && ptrow != nullptr) ? row0_pg(pre_static_pg[1])
-                                                                      : row0_of(t >> p.leaf_log2));
   wave_sync();
 
   const char* kb = reinterpret_cast<const char*>(reinterpret_cast<const T*>(p.k) + b * p.ksb + h * p.ksh + ds);
@@ -178,13 +182,19 @@ __device__ __forceinline__ void attn_query(const AttnParams& p, int n, int g, in
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int key = c * KPC + i * RPI + rg;
-      const int kt = key < nl ? key : 0;
-      const int r0 = s_row0[kt >> p.leaf_log2];
-      const int leafrow = r0 < 0 ? -1 : r0 + (kt & (leaf - 1));
-      const int ke = key - nl - nloc;
-      const int extrow = s_ext[(ke >= 0 && ke < next) ? ke : 0];
-      const int ownrow = own0 < 0 ? -1 : own0 + (key - nl);
-      row[i] = key < nl ? leafrow : (key < nl + nloc ? ownrow : (key < N ? extrow : -1));
+      if constexpr (CAND) {
+        const int pos = key < N ? p.cand[qi * p.KC + key] : -1;
+        const int r0 = (pos >= 0 && pos < p.Tk) ? row0_of(pos >> p.leaf_log2) : -1;
+        row[i] = r0 < 0 ? -1 : r0 + (pos & (leaf - 1));
+      } else {
+        const int kt = key < nl ? key : 0;
+        const int r0 = s_row0[kt >> p.leaf_log2];
+        const int leafrow = r0 < 0 ? -1 : r0 + (kt & (leaf - 1));
+        const int ke = key - nl - nloc;
+        const int extrow = s_ext[(ke >= 0 && ke < next) ? ke : 0];
+        const int ownrow = own0 < 0 ? -1 : own0 + (key - nl);
+        row[i] = key < nl ? leafrow : (key < nl + nloc ? ownrow : (key < N ? extrow : -1));
+      }
     }
 #pragma unroll
     for (int i = 0; i < NL; ++i) {

@@ -233,7 +233,7 @@ __device__ __noinline__ void task_seq_head(const StepPlan& P, const StepRun& R, 
   p.scale = P.scale;
   p.gsplit = 1;
   p.keys = R.keys ? R.keys + (int64_t)l * P.B * P.H : nullptr;
-  attn_query<bf16_t, D, true>(p, 0, 0, b, h, (int64_t)b * P.H + h, S.q, t, kid, nullptr, nk, P.n_tree, S.o,
+  attn_query<bf16_t, D, true, false>(p, 0, 0, b, h, (int64_t)b * P.H + h, S.q, t, kid, nullptr, nk, P.n_tree, S.o,
                                      att_smem);
   __syncthreads();
   TA_MARK(3);

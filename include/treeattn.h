@@ -241,9 +241,10 @@ int ta_sparse_attn_fwd(const void* q, const void* k, const void* v, int dtype,
  * with the last dimension contiguous; k, v rows 16-byte aligned.  D a multiple of 8 up to 256, B*H <= 65535.
  * dq is deterministic.  dk and dv:
  *   ws non-NULL (ta_sparse_attn_bwd_workspace_size bytes): written (every key row, zeros where no slot names
- *     it), each key's contributions added in a fixed order (queries ascending, slots ascending) -- bit for bit
- *     reproducible (the slots are sorted by key in ws first).  causal: every candidate position is at most its
- *     query's position (T == Tk); accepted for callers that know it, the result is the same.
+ *     it), each key's contributions added in an order that the slots alone fix -- bit for bit reproducible, at
+ *     every size (the slots are sorted by key in ws first, in parts where there are many: the workspace stays
+ *     within about 1 GiB unless one query has more than 2^26 slots).  causal: every candidate position is at most
+ *     its query's position (T == Tk); accepted for callers that know it, the result is the same.
  *   ws NULL: accumulated into with float32 atomic adds, as the reference's kernel does (zero them first); the
  *     summation order then depends on scheduling (reproducible to float32 rounding).
  */

@@ -68,6 +68,63 @@ def test_sorted_backward_matches_float64(T, Tk, KC, D, misaligned):
         assert (a.cpu().double() - w).abs().max().item() <= 1e-5 * max(1.0, w.abs().max().item())
 
 
+@pytest.mark.parametrize('T,Tk,KC', [
+    ((1 << 22) + 5, 300, 2),       # more queries than an entry can name: sorted in two parts
+    (20000, (1 << 21) + 33, 6),    # more keys than the buckets hold: summed in two parts
+    (16400, 5000, 4100),           # more slots than the workspace holds at a time, a chunk per query
+])
+def test_fixed_order_past_one_sort(T, Tk, KC):
+    """Sizes whose slots are sorted in several parts: the same bits every time (a key that every query names would
+    show another order), and the closed form in float64."""
+    print('case', T, Tk, KC, flush=True)
+    D, scale = 8, 1 / math.sqrt(8)
+    g = torch.Generator().manual_seed(T + KC)
+    q, do = (torch.randn(1, 1, T, D, generator=g) for _ in range(2))
+    k, v = (torch.randn(1, 1, Tk, D, generator=g) for _ in range(2))
+    cand = torch.randint(-2, Tk + 2, (1, 1, T, min(KC, 30)), generator=g)   # the slots after those are unused
+    cand[..., 0] = 0
+    out, lse, *want = _backward64(q, k, v, cand, scale, do)
+    q, k, v, do, out, lse = (x.float().to(DEV) for x in (q, k, v, do, out, lse))
+    cand = torch.nn.functional.pad(cand.int().to(DEV), (0, KC - cand.shape[-1]), value=-1)
+    got = K.sparse_attn_bwd(q, k, v, cand, scale, out, lse, do, deterministic=True)
+    again = K.sparse_attn_bwd(q, k, v, cand, scale, out, lse, do, deterministic=True)
+    # a key's list is added in up to 2050 parts (one per tile of 2048 entries) whose running sum is rounded each time:
+    # about sqrt(2050) * 2^-24 = 2.7e-6 of the largest value
+    for a, b, w in zip(got, again, want):
+        assert torch.equal(a, b)
+        assert (a.cpu().double() - w).abs().max().item() <= 1e-5 * max(1.0, w.abs().max().item())
+
+
+def test_pairs_in_groups_equal_pairs_alone():
+    """More slots than the workspace holds at a time, over the (sequence, head) pairs: each pair's gradients are bit for
+    bit those of a call on it alone."""
+    B, H, T, D, KC = 1, 36, 500, 8, 4000
+    g = torch.Generator(device=DEV).manual_seed(9)
+    q, k, v, do, out = (torch.randn(B, H, T, D, generator=g, device=DEV) for _ in range(5))
+    cand = torch.randint(-3 * T, T, (B, H, T, KC), generator=g, device=DEV, dtype=torch.int32)
+    lse = torch.full((B, H, T), 7.0, device=DEV)   # any values do: what is compared is the same sums
+    got = K.sparse_attn_bwd(q, k, v, cand, 0.3, out, lse, do, deterministic=True)
+    for h in (0, 28, 29, 35):   # 29 pairs are sorted together
+        part = [x[:, h:h + 1] for x in (q, k, v, cand, out, lse, do)]
+        alone = K.sparse_attn_bwd(*part[:4], 0.3, *part[4:], deterministic=True)
+        assert all(torch.equal(a[:, h:h + 1], b) for a, b in zip(got, alone))
+
+
+def test_no_slots_with_a_workspace_gives_zeros():
+    """No candidate slots: dq, dk and dv are written as zeros (the entry point itself; the wrapper takes no workspace)."""
+    from treeattn_amd import _lib as L
+    B, H, T, Tk, D = 2, 3, 5, 700, 24
+    q, o, do = (torch.randn(B, H, T, D, device=DEV) for _ in range(3))
+    k, v = (torch.randn(B, H, Tk, D, device=DEV) for _ in range(2))
+    dq, dk, dv = (torch.full_like(x, 7.0) for x in (q, k, v))
+    cand, ws = torch.zeros(1, dtype=torch.int32, device=DEV), torch.zeros(4, device=DEV)
+    lse = torch.zeros(B, H, T, device=DEV)
+    L.call('ta_sparse_attn_bwd', *(L.ptr(x) for x in (q, k, v, o, do)), L.F32, *L.rows3(q), *L.rows3(k), *L.rows3(v),
+           *L.rows3(o), *L.rows3(do), L.ptr(cand), L.ptr(lse), B, H, T, Tk, 0, D, 1.0, L.ptr(dq), L.ptr(dk), L.ptr(dv),
+           L.ptr(ws), 0, L.stream())
+    assert all(bool((x == 0).all()) for x in (dq, dk, dv))
+
+
 @pytest.mark.parametrize('dtype,T,H,D', [(torch.float32, 130, 3, 16), (torch.float16, 77, 2, 64), (torch.bfloat16, 1, 2, 128),
                                          (torch.float16, 33, 1, 64), (torch.float16, 50, 2, 32)])
 @pytest.mark.parametrize('case', ['views', 'offset', 'broadcast'])

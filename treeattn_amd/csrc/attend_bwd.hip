@@ -9,14 +9,15 @@
 // group, and dq takes the key row that is still in registers.  dk and dv then take one of two routes:
 //  * with a workspace (the Python binding's default while its bound holds): every valid slot's ds and p are written
 //    there, the slots are sorted by key in a stable order (queries ascending, slots ascending) and
-//    bwd_keys_kernel adds each key's contributions from its own consecutive list.  The order of the additions is
-//    fixed: dk and dv are bit-reproducible.
+//    bwd_keys_kernel adds each key's contributions from its own consecutive list.  Which entries a lane adds, and
+//    how the lanes' and wavefronts' parts are added, follows from the list alone: dk and dv are bit-reproducible.
 //  * without one, each slot's dk and dv rows receive float32 atomic adds (the reference's scheme, whose order
 //    depends on scheduling: reproducible to float32 rounding only).
 //
 // The sort is one stable most-significant-digit pass over chunks of queries (bwd_count_kernel, bwd_scan_kernel,
 // bwd_scatter_kernel) into at most 2048 buckets of 16 (or more) consecutive keys; bwd_keys_kernel lists a bucket's
-// entries key by key in LDS.  The cost is linear in the slots.  Scanning all candidate rows once per block of keys
+// entries key by key in LDS.  The cost is linear in the slots.  Past 2^26 slots, 2^22 queries or 2^21 keys the pairs
+// and queries are sorted, and the keys summed, in parts one after another, which keeps the order.  Scanning all candidate rows once per block of keys
 // instead (one wavefront per block, a serial chain over the queries, quadratic in T) took 6.2 ms of the 7.0 ms
 // forward and backward of a (2, 6, 4096, 64) float16 layer with 52 candidates a row (12 valid); this takes 0.13 ms:
 // count 8, scan 14, scatter 18 and keys 90 us.  What is left in the key kernel is latency (about 8 us per bucket, six
@@ -34,13 +35,16 @@ struct BwdParams {
   const float* lse;      // (B,H,T) contiguous
   void* dq;              // (B,H,T,D) rows, input dtype
   float *dk, *dv;        // (B,H,Tk,D) rows, float32: accumulated into (atomics) or written (workspace)
-  float2* dsp;           // (B,H,T,KC) per-slot (ds, p), written where the slot is valid (the sorted route), or null
-  uint2* ent;            // (B,H,T*KC) sorted entries: slot index, query << kLowBits | key within its bucket
-  int32_t* cnt;          // per (b,h): [bucket][chunk] counts, then starts; one more word: the number of entries
+  // the sorted route's workspace, for the `pairs` (b,h) from bh0 on and their queries [t0, t0 + Ts):
+  float2* dsp;           // (pairs,Ts,KC) per-slot (ds, p), written where the slot is valid, or null
+  uint2* ent;            // (pairs,Ts*KC) sorted entries: slot index, query << kLowBits | key within its bucket
+  int32_t* cnt;          // per pair: [bucket][chunk] counts, then starts; one more word: the number of entries
   int B, H, T, Tk, KC, D;
+  int bh0, t0, Ts;       // this launch's pairs and queries
+  int j0, Tj;            // the keys being summed: [j0, j0 + Tj)
   float scale;
   int rows_al;           // q, o and do rows, dq, dk and dv are 16-byte aligned
-  int CQ, NC;            // queries per chunk, chunks
+  int CQ, NC;            // queries per chunk, chunks of the Ts queries
   int wlog, NB;          // log2 of a bucket's keys, buckets
   int64_t gq[3], gk[3], gv[3];   // strides (b, h, row) of dq, dk, dv
 };
@@ -52,6 +56,7 @@ constexpr int kChunkSlots = 4096;     // slots per chunk (at least one query)
 constexpr int kBwdWaves = 4;          // wavefronts of the query, count and scatter kernels
 constexpr int kKeyWaves = 8;
 constexpr int kTile = 2048;           // entries sorted in LDS at a time
+constexpr int64_t kSortSlots = 1 << 26;
 constexpr int kHeavy = 96;            // a key with more entries in a tile is shared by the workgroup's wavefronts
 
 // Lanes per row: the power of two of 8-dimension slices that covers D (lanes past D hold zeros).
@@ -118,8 +123,9 @@ __global__ __launch_bounds__(kWave * kBwdWaves) void bwd_query_kernel(BwdParams 
   constexpr int G = kWave / L;   // slots worked on together
   __shared__ int s_row[kBwdWaves][kWave], s_slot[kBwdWaves][kWave];
   const int lane = lane_id(), wv = wave_id();
-  const int t = blockIdx.x * kBwdWaves + wv, bh = blockIdx.y;
-  if (t >= p.T) return;   // a whole wavefront leaves; no workgroup barrier follows
+  const int ts = blockIdx.x * kBwdWaves + wv;
+  if (ts >= p.Ts) return;   // a whole wavefront leaves; no workgroup barrier follows
+  const int t = p.t0 + ts, bh = p.bh0 + blockIdx.y;
   const int b = bh / p.H, h = bh - b * p.H;
   const int D = p.D;
   const int g = lane / L, d0 = (lane % L) * 8;
@@ -129,6 +135,7 @@ __global__ __launch_bounds__(kWave * kBwdWaves) void bwd_query_kernel(BwdParams 
   const T* vb = reinterpret_cast<const T*>(p.v) + b * p.vsb + h * p.vsh + d0;
   const int64_t row = (int64_t)bh * p.T + t;
   const int32_t* cr = p.cand + row * p.KC;
+  float2* dsp = p.dsp + ((int64_t)blockIdx.y * p.Ts + ts) * p.KC;
   const float lse = p.lse[row];
   float qf[8], df[8], of[8];
   load8(reinterpret_cast<const T*>(p.q) + b * p.qsb + h * p.qsh + (int64_t)t * p.qst + d0, in, al, qf);
@@ -174,7 +181,7 @@ __global__ __launch_bounds__(kWave * kBwdWaves) void bwd_query_kernel(BwdParams 
       for (int e = 0; e < 8; ++e) dq[e] += ds * kf[e];
       if (live) {
         if (p.dsp != nullptr) {
-          if (d0 == 0) p.dsp[row * p.KC + s_slot[wv][i]] = make_float2(ds, pw);
+          if (d0 == 0) dsp[s_slot[wv][i]] = make_float2(ds, pw);
         } else if (in) {
           float* dkr = p.dk + b * p.gk[0] + h * p.gk[1] + jr * p.gk[2] + d0;
           float* dvr = p.dv + b * p.gv[0] + h * p.gv[1] + jr * p.gv[2] + d0;
@@ -194,11 +201,20 @@ __global__ __launch_bounds__(kWave * kBwdWaves) void bwd_query_kernel(BwdParams 
 }
 
 // ---------------------------------------------------------------------------------- sorting the slots by key
-// A chunk's slots are consecutive: queries [ch * CQ, ...), KC slots each.
+// A chunk's slots are consecutive: queries [ch * CQ, ...) of the Ts, KC slots each.
 __device__ __forceinline__ void chunk_range(const BwdParams& p, int ch, int& s0, int& s1) {
-  const int t0 = ch * p.CQ, t1 = t0 + p.CQ < p.T ? t0 + p.CQ : p.T;
+  const int t0 = ch * p.CQ, t1 = t0 + p.CQ < p.Ts ? t0 + p.CQ : p.Ts;
   s0 = t0 * p.KC;
   s1 = t1 * p.KC;
+}
+
+// A candidate's key counted from the first one being summed: below Tj where it is one of them (unused slots, which
+// are negative, wrap to the top).
+__device__ __forceinline__ uint32_t key_of(const BwdParams& p, int32_t cand) { return (uint32_t)cand - (uint32_t)p.j0; }
+
+// The candidate slots of pair `pair`'s queries from t0 on.
+__device__ __forceinline__ const int32_t* pair_slots(const BwdParams& p, int pair) {
+  return p.cand + ((int64_t)(p.bh0 + pair) * p.T + p.t0) * p.KC;
 }
 
 __global__ __launch_bounds__(kWave * kBwdWaves) void bwd_count_kernel(BwdParams p) {
@@ -208,10 +224,10 @@ __global__ __launch_bounds__(kWave * kBwdWaves) void bwd_count_kernel(BwdParams 
   __syncthreads();
   int s0, s1;
   chunk_range(p, ch, s0, s1);
-  const int32_t* cr = p.cand + (int64_t)bh * p.T * p.KC;
+  const int32_t* cr = pair_slots(p, bh);
   for (int s = s0 + threadIdx.x; s < s1; s += blockDim.x) {
-    const int j = cr[s];
-    if (j >= 0 && j < p.Tk) atomicAdd(&s_n[j >> p.wlog], 1);
+    const uint32_t j = key_of(p, cr[s]);
+    if (j < (uint32_t)p.Tj) atomicAdd(&s_n[j >> p.wlog], 1);
   }
   __syncthreads();
   int32_t* cnt = p.cnt + (int64_t)bh * ((int64_t)p.NB * p.NC + 1);
@@ -283,10 +299,10 @@ __global__ __launch_bounds__(kWave * kBwdWaves) void bwd_scatter_kernel(BwdParam
   chunk_range(p, ch, s0, s1);
   const int part = (s1 - s0 + kBwdWaves - 1) / kBwdWaves;
   const int a0 = s0 + wv * part, a1 = a0 + part < s1 ? a0 + part : s1;
-  const int32_t* cr = p.cand + (int64_t)bh * p.T * p.KC;
+  const int32_t* cr = pair_slots(p, bh);
   for (int s = a0 + lane; s < a1; s += kWave) {
-    const int j = cr[s];
-    if (j >= 0 && j < p.Tk) atomicAdd(&mine[j >> p.wlog], 1);
+    const uint32_t j = key_of(p, cr[s]);
+    if (j < (uint32_t)p.Tj) atomicAdd(&mine[j >> p.wlog], 1);
   }
   __syncthreads();
   const int32_t* cnt = p.cnt + (int64_t)bh * ((int64_t)p.NB * p.NC + 1);
@@ -300,21 +316,21 @@ __global__ __launch_bounds__(kWave * kBwdWaves) void bwd_scatter_kernel(BwdParam
     }
   }
   __syncthreads();
-  uint2* ent = p.ent + (int64_t)bh * p.T * p.KC;
+  uint2* ent = p.ent + (int64_t)bh * p.Ts * p.KC;
   const int bits = 32 - __clz(p.NB - 1 | 1);
   const uint64_t below = (1ull << lane) - 1;
-  const int low = (1 << p.wlog) - 1;
+  const uint32_t low = (1u << p.wlog) - 1;
   for (int sb = a0; sb < a1; sb += kWave) {
     const int s = sb + lane;
-    const int j = s < a1 ? cr[s] : -1;
-    const bool ok = j >= 0 && j < p.Tk;
-    const int d = ok ? j >> p.wlog : 0;
+    const uint32_t j = s < a1 ? key_of(p, cr[s]) : ~0u;
+    const bool ok = j < (uint32_t)p.Tj;
+    const int d = ok ? (int)(j >> p.wlog) : 0;
     const uint64_t m = same_digit(d, ok, bits);
     int at = 0;
     if (ok) at = mine[d] + __popcll(m & below);
     wave_sync();
     if (ok) {
-      ent[at] = make_uint2((uint32_t)s, (uint32_t)(s / p.KC) << kLowBits | (uint32_t)(j & low));
+      ent[at] = make_uint2((uint32_t)s, (uint32_t)(s / p.KC) << kLowBits | (j & low));
       if ((m >> lane) == 1) mine[d] = at + 1;   // the last lane of the digit
     }
     wave_sync();
@@ -382,7 +398,7 @@ __device__ __forceinline__ void key_part(const BwdParams& p, const T* qb, const 
 // per round every wavefront takes one key, lists the tile's entries of that key (ballots over the tile, which keeps
 // their order) and adds their contributions, 64 / L entries at a time (the q and do rows in whole lines, the groups'
 // partial sums in a fixed order).  A key that many queries name (the sink) is shared by all wavefronts, their parts
-// added in order.  Each row is written by the first tile and added to by later ones.
+// added in order.  Each row is written by the first tile of the first queries and added to by later ones.
 template <typename T, int L, bool VEC>
 __global__ __launch_bounds__(kWave * kKeyWaves, 4) void bwd_keys_kernel(BwdParams p) {
   __shared__ uint2 s_e[kTile];
@@ -391,20 +407,20 @@ __global__ __launch_bounds__(kWave * kKeyWaves, 4) void bwd_keys_kernel(BwdParam
   __shared__ float s_part[kKeyWaves][2][L * 8];
   const int lane = lane_id(), wv = wave_id(), tid = threadIdx.x;
   const int bh = blockIdx.x, bk = blockIdx.y;   // first buckets first: they hold the sink, the longest list
-  const int b = bh / p.H, h = bh - b * p.H;
+  const int b = (p.bh0 + bh) / p.H, h = p.bh0 + bh - b * p.H;
   const int D = p.D;
   const int g = lane / L, d0 = (lane % L) * 8;
   const bool in = d0 < D;
-  const int j0 = bk << p.wlog;
+  const int j0 = p.j0 + (bk << p.wlog);
   const int W = 1 << p.wlog;
-  const int nk = p.Tk - j0 < W ? p.Tk - j0 : W;
+  const int nk = p.j0 + p.Tj - j0 < W ? p.j0 + p.Tj - j0 : W;
   const int32_t* cnt = p.cnt + (int64_t)bh * ((int64_t)p.NB * p.NC + 1);
   const int first = cnt[(int64_t)bk * p.NC], last = cnt[(int64_t)(bk + 1) * p.NC];
-  const uint2* ent = p.ent + (int64_t)bh * p.T * p.KC;
-  const float2* dsp = p.dsp + (int64_t)bh * p.T * p.KC;
+  const uint2* ent = p.ent + (int64_t)bh * p.Ts * p.KC;
+  const float2* dsp = p.dsp + (int64_t)bh * p.Ts * p.KC;
   const int dl = in ? d0 : 0;   // lanes past the row read its first slice and write nothing
-  const T* qb = reinterpret_cast<const T*>(p.q) + b * p.qsb + h * p.qsh + dl;
-  const T* db = reinterpret_cast<const T*>(p.dout) + b * p.dsb + h * p.dsh + dl;
+  const T* qb = reinterpret_cast<const T*>(p.q) + b * p.qsb + h * p.qsh + p.t0 * p.qst + dl;
+  const T* db = reinterpret_cast<const T*>(p.dout) + b * p.dsb + h * p.dsh + p.t0 * p.dst + dl;
   float* dkb = p.dk + b * p.gk[0] + h * p.gk[1] + j0 * p.gk[2];
   float* dvb = p.dv + b * p.gv[0] + h * p.gv[1] + j0 * p.gv[2];
   const uint64_t below = (1ull << lane) - 1;
@@ -427,7 +443,7 @@ __global__ __launch_bounds__(kWave * kKeyWaves, 4) void bwd_keys_kernel(BwdParam
   float dk[8], dv[8];
   int at = first;
   do {
-    const bool fresh = at == first;
+    const bool fresh = at == first && p.t0 == 0;
     const int n = last - at < kTile ? last - at : kTile;
     for (int i = tid; i < n; i += kWave * kKeyWaves) s_e[i] = ent[at + i];
     __syncthreads();
@@ -485,48 +501,80 @@ __global__ void bwd_zero_kernel(float* a, float* b, int64_t n) {
     a[i] = b[i] = 0.0f;
 }
 
-// Chunks, buckets and workspace words (float32) of the sorted route.
+// How the sorted route is cut: `pairs` (b,h) and Ts queries of each at a time, so that the workspace stays within
+// kSortSlots slots (1 GiB; more only where a single query has more slots) and a slot and a query fit an entry's words.
+// The pieces of a key's list come in order of the queries, so the cut does not disturb the fixed order of the sums.
 struct BwdPlan {
-  int CQ, NC, wlog, NB;
-  bool ok;   // the slot and query indices fit the entries
+  int pairs, Ts;
+  int CQ, NC;            // queries per chunk, chunks
+  int64_t slots, words;  // of a pair: slots of the Ts queries, words of the counts
 };
 
-static BwdPlan bwd_plan(int T, int Tk, int KC) {
+static BwdPlan bwd_plan(int B, int H, int T, int KC) {
   BwdPlan r;
+  const int64_t fit = kSortSlots / KC > 1 ? kSortSlots / KC : 1;
+  const int64_t most = fit < (1 << (32 - kLowBits)) ? fit : 1 << (32 - kLowBits);
+  r.Ts = (int)(T < most ? T : most);
   r.CQ = KC >= kChunkSlots ? 1 : kChunkSlots / KC;
-  r.NC = (T + r.CQ - 1) / r.CQ;
-  r.wlog = 4;   // 16 keys: two per wavefront of the key kernel
-  while (((Tk - 1) >> r.wlog) + 1 > kMaxBuckets) ++r.wlog;
-  r.NB = ((Tk - 1) >> r.wlog) + 1;
-  r.ok = (int64_t)T * KC < (1ll << 31) - (1 << 16) && T <= (1 << (32 - kLowBits)) && r.wlog <= kLowBits;
+  r.NC = (r.Ts + r.CQ - 1) / r.CQ;
+  r.slots = (int64_t)r.Ts * KC;
+  r.words = (int64_t)kMaxBuckets * r.NC + 1;
+  const int64_t bh = (int64_t)B * H, together = kSortSlots / (r.slots + r.words / 4 + 1);
+  r.pairs = (int)(bh < together ? bh : together > 1 ? together : 1);
   return r;
 }
 
 template <typename T, int L>
-static void launch_bwd(const BwdParams& p, bool sorted, hipStream_t st) {
+static void launch_query(const BwdParams& p, int pairs, hipStream_t st) {
+  hipLaunchKernelGGL((bwd_query_kernel<T, L>), dim3((unsigned)((p.Ts + kBwdWaves - 1) / kBwdWaves), (unsigned)pairs),
+                     dim3(kWave * kBwdWaves), 0, st, p);
+}
+
+template <typename T, int L>
+static void launch_bwd(BwdParams p, const BwdPlan* pl, hipStream_t st) {
+  const int bh = p.B * p.H;
+  if (pl == nullptr) {   // atomic adds
+    launch_query<T, L>(p, bh, st);
+    return;
+  }
   const dim3 block(kWave * kBwdWaves);
-  const unsigned bh = (unsigned)(p.B * p.H);
-  hipLaunchKernelGGL((bwd_query_kernel<T, L>), dim3((unsigned)((p.T + kBwdWaves - 1) / kBwdWaves), bh), block, 0, st, p);
-  if (!sorted) return;
-  hipLaunchKernelGGL(bwd_count_kernel, dim3((unsigned)p.NC, bh), block, 0, st, p);
-  hipLaunchKernelGGL(bwd_scan_kernel, dim3(bh), dim3(1024), 0, st, p);
-  hipLaunchKernelGGL(bwd_scatter_kernel, dim3((unsigned)p.NC, bh), block, 0, st, p);
-  const dim3 kgrid(bh, (unsigned)p.NB), kblock(kWave * kKeyWaves);
-  if (p.rows_al)
-    hipLaunchKernelGGL((bwd_keys_kernel<T, L, true>), kgrid, kblock, 0, st, p);
-  else
-    hipLaunchKernelGGL((bwd_keys_kernel<T, L, false>), kgrid, kblock, 0, st, p);
+  constexpr int kMaxKeys = kMaxBuckets << kLowBits;   // sorted at a time
+  for (p.bh0 = 0; p.bh0 < bh; p.bh0 += pl->pairs) {
+    const int pairs = bh - p.bh0 < pl->pairs ? bh - p.bh0 : pl->pairs;
+    for (int64_t t0 = 0; t0 < p.T; t0 += pl->Ts) {
+      p.t0 = (int)t0;
+      p.Ts = p.T - p.t0 < pl->Ts ? p.T - p.t0 : pl->Ts;
+      p.NC = (p.Ts + p.CQ - 1) / p.CQ;
+      launch_query<T, L>(p, pairs, st);
+      for (int64_t j0 = 0; j0 < p.Tk; j0 += kMaxKeys) {
+        p.j0 = (int)j0;
+        p.Tj = p.Tk - p.j0 < kMaxKeys ? p.Tk - p.j0 : kMaxKeys;
+        p.wlog = 4;   // 16 keys: two per wavefront of the key kernel
+        while (((p.Tj - 1) >> p.wlog) + 1 > kMaxBuckets) ++p.wlog;
+        p.NB = ((p.Tj - 1) >> p.wlog) + 1;
+        const dim3 cgrid((unsigned)p.NC, (unsigned)pairs);
+        hipLaunchKernelGGL(bwd_count_kernel, cgrid, block, 0, st, p);
+        hipLaunchKernelGGL(bwd_scan_kernel, dim3((unsigned)pairs), dim3(1024), 0, st, p);
+        hipLaunchKernelGGL(bwd_scatter_kernel, cgrid, block, 0, st, p);
+        const dim3 kgrid((unsigned)pairs, (unsigned)p.NB), kblock(kWave * kKeyWaves);
+        if (p.rows_al)
+          hipLaunchKernelGGL((bwd_keys_kernel<T, L, true>), kgrid, kblock, 0, st, p);
+        else
+          hipLaunchKernelGGL((bwd_keys_kernel<T, L, false>), kgrid, kblock, 0, st, p);
+      }
+    }
+  }
 }
 
 template <typename T>
-static void launch_bwd_d(const BwdParams& p, bool sorted, hipStream_t st) {
+static void launch_bwd_d(const BwdParams& p, const BwdPlan* pl, hipStream_t st) {
   switch (bwd_lanes(p.D)) {
-    case 1: launch_bwd<T, 1>(p, sorted, st); break;
-    case 2: launch_bwd<T, 2>(p, sorted, st); break;
-    case 4: launch_bwd<T, 4>(p, sorted, st); break;
-    case 8: launch_bwd<T, 8>(p, sorted, st); break;
-    case 16: launch_bwd<T, 16>(p, sorted, st); break;
-    default: launch_bwd<T, 32>(p, sorted, st); break;
+    case 1: launch_bwd<T, 1>(p, pl, st); break;
+    case 2: launch_bwd<T, 2>(p, pl, st); break;
+    case 4: launch_bwd<T, 4>(p, pl, st); break;
+    case 8: launch_bwd<T, 8>(p, pl, st); break;
+    case 16: launch_bwd<T, 16>(p, pl, st); break;
+    default: launch_bwd<T, 32>(p, pl, st); break;
   }
 }
 
@@ -561,33 +609,40 @@ static int sparse_attn_bwd_impl(const void* q, const void* k, const void* v, con
     return TA_ERR_UNSUPPORTED;
   }
   // rows of q, o, dout, dq, dk and dv are moved 8 elements at a time where all are aligned, else one by one
-  const int al = !(((uintptr_t)q | (uintptr_t)o | (uintptr_t)dout | (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) % 16 || (qsb * es) % 16 || (qsh * es) % 16 ||
-                   (qst * es) % 16 || (osb * es) % 16 || (osh * es) % 16 || (ost * es) % 16 || (dsb * es) % 16 ||
-                   (dsh * es) % 16 || (dst * es) % 16 || ((gs[0] | gs[1] | gs[2]) * es) % 16 ||
+  const int al = !(((uintptr_t)q | (uintptr_t)o | (uintptr_t)dout | (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) % 16 ||
+                   (qsb * es) % 16 || (qsh * es) % 16 || (qst * es) % 16 || (osb * es) % 16 || (osh * es) % 16 ||
+                   (ost * es) % 16 || (dsb * es) % 16 || (dsh * es) % 16 || (dst * es) % 16 ||
+                   ((gs[0] | gs[1] | gs[2]) * es) % 16 ||
                    ((gs[3] | gs[4] | gs[5] | gs[6] | gs[7] | gs[8]) * 4) % 16);
-  BwdParams p{q, k, v, o, dout, qsb, qsh, qst, ksb, ksh, kst, vsb, vsh, vst, osb, osh, ost, dsb, dsh, dst,
-              cand, lse, dq, dk, dv, nullptr, nullptr, nullptr, B, H, T, Tk, KC, D, scale, al, 0, 0, 0, 0, {gs[0], gs[1], gs[2]}, {gs[3], gs[4], gs[5]}, {gs[6], gs[7], gs[8]}};
+  BwdParams p{};
+  p.q = q, p.k = k, p.v = v, p.o = o, p.dout = dout;
+  p.qsb = qsb, p.qsh = qsh, p.qst = qst, p.ksb = ksb, p.ksh = ksh, p.kst = kst, p.vsb = vsb, p.vsh = vsh, p.vst = vst;
+  p.osb = osb, p.osh = osh, p.ost = ost, p.dsb = dsb, p.dsh = dsh, p.dst = dst;
+  p.cand = cand, p.lse = lse, p.dq = dq, p.dk = dk, p.dv = dv;
+  p.B = B, p.H = H, p.T = T, p.Tk = Tk, p.KC = KC, p.D = D, p.Ts = T;
+  p.scale = scale;
+  p.rows_al = al;
+  for (int i = 0; i < 3; ++i) p.gq[i] = gs[i], p.gk[i] = gs[3 + i], p.gv[i] = gs[6 + i];
   hipStream_t st = (hipStream_t)stream;
-  bool sorted = ws != nullptr && KC > 0;
+  BwdPlan pl;
+  const bool sorted = ws != nullptr && KC > 0;
   if (sorted) {
-    const BwdPlan pl = bwd_plan(T, Tk, KC);
-    const int64_t slots = (int64_t)B * H * T * KC;
-    sorted = pl.ok;
+    pl = bwd_plan(B, H, T, KC);
+    const int64_t slots = pl.pairs * pl.slots;
     p.dsp = reinterpret_cast<float2*>(ws);
     p.ent = reinterpret_cast<uint2*>(ws + 2 * slots);
     p.cnt = reinterpret_cast<int32_t*>(ws + 4 * slots);
-    p.CQ = pl.CQ, p.NC = pl.NC, p.wlog = pl.wlog, p.NB = pl.NB;
-  }
-  if (ws != nullptr && !sorted) {   // indices past the entries' 32 bits, or no slots: atomic adds into cleared rows
-    p.dsp = nullptr;
+    p.CQ = pl.CQ;
+  } else if (ws != nullptr) {   // no slots: every row is zero
     const int64_t n = (int64_t)B * H * Tk * D;
     const int64_t wgs = (n + 255) / 256;
     hipLaunchKernelGGL(bwd_zero_kernel, dim3((unsigned)(wgs < 4096 ? wgs : 4096)), dim3(256), 0, st, dk, dv, n);
   }
+  const BwdPlan* plan = sorted ? &pl : nullptr;
   switch (dtype) {
-    case TA_F32: launch_bwd_d<float>(p, sorted, st); break;
-    case TA_F16: launch_bwd_d<f16_t>(p, sorted, st); break;
-    default: launch_bwd_d<bf16_t>(p, sorted, st); break;
+    case TA_F32: launch_bwd_d<float>(p, plan, st); break;
+    case TA_F16: launch_bwd_d<f16_t>(p, plan, st); break;
+    default: launch_bwd_d<bf16_t>(p, plan, st); break;
   }
   return check_launch("ta_sparse_attn_bwd");
 }
@@ -620,10 +675,9 @@ extern "C" int ta_sparse_attn_bwd_strided(const void* q, const void* k, const vo
 }
 
 // Workspace of the sorted dk / dv route of ta_sparse_attn_bwd: per-slot (ds, p), the sorted entries, and the counts of
-// at most kMaxBuckets buckets per chunk of queries (whatever the number of keys).
+// at most kMaxBuckets buckets per chunk of queries (whatever the number of keys), for what bwd_plan sorts at a time.
 extern "C" int64_t ta_sparse_attn_bwd_workspace_size(int B, int H, int T, int KC) {
   if (B <= 0 || H <= 0 || T <= 0 || KC <= 0) return 0;
-  const BwdPlan pl = bwd_plan(T, 1, KC);
-  const int64_t bh = (int64_t)B * H;
-  return (4 * bh * T * KC + bh * ((int64_t)kMaxBuckets * pl.NC + 1)) * (int64_t)sizeof(float);
+  const BwdPlan pl = bwd_plan(B, H, T, KC);
+  return pl.pairs * (4 * pl.slots + pl.words) * (int64_t)sizeof(float);
 }

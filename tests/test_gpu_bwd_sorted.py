@@ -150,3 +150,27 @@ def test_strided_rows_equal_contiguous(dtype, T, H, D, case):
     tol = {torch.float32: 1e-5, torch.float16: 2e-3, torch.bfloat16: 1.6e-2}[dtype]
     for a, b in zip(K.sparse_attn_bwd(q, k, v, cand, 0.125, out, lse, do, deterministic=False), want):
         assert (a.float() - b.float()).abs().max().item() <= tol * max(1.0, b.float().abs().max().item())
+
+
+def test_atomic_route_adds_whole_lines():
+    """The atomic adds go to consecutive dimensions from consecutive lanes: with lanes 32 bytes apart this call took 13.4
+    times the sorted route's; consecutive ones take about 3 times (337 against 109 us at 52 slots, a quarter of them
+    valid, float16)."""
+    B, H, T, D, KC = 2, 6, 2048, 64, 13
+    g = torch.Generator(device=DEV).manual_seed(5)
+    q, k, v, do = (torch.randn(B, H, T, D, generator=g, device=DEV) for _ in range(4))
+    cand = torch.randint(0, T, (B, H, T, KC), generator=g, device=DEV, dtype=torch.int32)
+    out, lse = K.sparse_attn_fwd(q, k, v, cand, 0.125)
+
+    def us(det):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = math.inf
+        for _ in range(6):
+            a.record()
+            for _ in range(4):
+                K.sparse_attn_bwd(q, k, v, cand, 0.125, out, lse, do, deterministic=det)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+    assert us(False) < 9 * us(True)

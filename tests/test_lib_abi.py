@@ -85,6 +85,20 @@ def test_product_refuses_cpu_tensors():
         kernels.gather_dot(q, q, torch.zeros(1, 1, 4, 2, dtype=torch.long), 1.0)
 
 
+def test_backward_workspace_is_bounded():
+    """The sorted backward's workspace: 16 bytes a slot and the counts of at most 256 chunks of queries, for what is
+    sorted at a time -- at most 2^26 slots, or one query's."""
+    from treeattn_amd import _lib
+    size = _lib.lib().ta_sparse_attn_bwd_workspace_size
+    counts = (2048 * 256 + 1) * 4
+    for B, H, T, KC in [(1, 1, 1, 1), (2, 6, 4096, 52), (1, 1, 262144, 52), (1, 1, 16384, 2100), (1, 3, 300, 5000)]:
+        assert 0 < size(B, H, T, KC) - 16 * B * H * T * KC <= B * H * counts, (B, H, T, KC)
+    for B, H, T, KC in [(4096, 12, 256, 52), (1, 16, 16384, 2100), (65535, 1, 16, 16), (1, 1, (1 << 22) + 5, 600)]:
+        assert size(B, H, T, KC) <= (1 << 30) + counts, (B, H, T, KC)
+    assert size(1, 1, 3, 1 << 27) <= (16 << 27) + counts
+    assert size(0, 1, 8, 8) == size(1, 1, 0, 8) == size(1, 1, 8, 0) == 0
+
+
 def test_backward_route_choice():
     """The default dk/dv route: the fixed-order (bit-reproducible) scan while its candidate-row reads stay within
     DKDV_SCAN_LIMIT, the atomic adds beyond (the scan is quadratic in T).  Causal scans skip the queries before a

@@ -53,6 +53,10 @@ constexpr int kBwdMaxD = 256;
 constexpr int kLowBits = 10;          // bits of the key within its bucket
 constexpr int kMaxBuckets = 2048;
 constexpr int kChunkSlots = 4096;     // slots per chunk (at least one query)
+// At most this many chunks, larger ones past it (from about 20,000 queries of 52 slots on): the scan of a pair's counts
+// is one workgroup's, and with chunks of 4096 slots throughout it grew with the square of the queries: 6.2 of the
+// 17.7 ms of (1, 1, 262144, 64), against 0.5 of 12.1
+constexpr int kMaxChunks = 256;
 constexpr int kBwdWaves = 4;          // wavefronts of the query, count and scatter kernels
 constexpr int kKeyWaves = 8;
 constexpr int kTile = 2048;           // entries sorted in LDS at a time
@@ -537,6 +541,7 @@ static BwdPlan bwd_plan(int B, int H, int T, int KC) {
   const int64_t most = fit < (1 << (32 - kLowBits)) ? fit : 1 << (32 - kLowBits);
   r.Ts = (int)(T < most ? T : most);
   r.CQ = KC >= kChunkSlots ? 1 : kChunkSlots / KC;
+  if (r.CQ < (r.Ts + kMaxChunks - 1) / kMaxChunks) r.CQ = (r.Ts + kMaxChunks - 1) / kMaxChunks;
   r.NC = (r.Ts + r.CQ - 1) / r.CQ;
   r.slots = (int64_t)r.Ts * KC;
   r.words = (int64_t)kMaxBuckets * r.NC + 1;

@@ -174,3 +174,18 @@ def test_atomic_route_adds_whole_lines():
             best = min(best, a.elapsed_time(b))
         return best
     assert us(False) < 9 * us(True)
+
+
+def test_default_is_the_fixed_order_at_training_lengths():
+    """The default at a long training sequence: the fixed order's bits (atomic adds to the key that every query names
+    would differ between runs)."""
+    B, H, T, D, KC = 1, 6, 32768, 64, 52
+    g = torch.Generator(device=DEV).manual_seed(6)
+    q, k, v, do = (torch.randn(B, H, T, D, generator=g, device=DEV) for _ in range(4))
+    cand = torch.randint(-3 * T, T, (B, H, T, KC), generator=g, device=DEV, dtype=torch.int32)
+    cand[..., 0] = 0
+    out, lse = K.sparse_attn_fwd(q, k, v, cand, 0.125)
+    got = K.sparse_attn_bwd(q, k, v, cand, 0.125, out, lse, do)
+    for det in (None, True):
+        again = K.sparse_attn_bwd(q, k, v, cand, 0.125, out, lse, do, deterministic=det)
+        assert all(torch.equal(a, b) for a, b in zip(got, again))

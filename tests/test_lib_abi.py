@@ -100,15 +100,12 @@ def test_backward_workspace_is_bounded():
 
 
 def test_backward_route_choice():
-    """The default dk/dv route: the fixed-order (bit-reproducible) scan while its candidate-row reads stay within
-    DKDV_SCAN_LIMIT, the atomic adds beyond (the scan is quadratic in T).  Causal scans skip the queries before a
-    key block: sum over blocks of (T - block start) rows."""
+    """The default dk/dv route: the fixed (bit-reproducible) order up to SORTED_MAX_POSITIONS queries and keys, the atomic
+    adds past it, whatever the number of pairs and slots (the workspace is bounded)."""
     from treeattn_amd import kernels as K
-    # T = 512, D = 64 (blocks of 64 keys), KC = 100: 8 blocks x 512 rows, or 512 + 448 + ... + 64 causally
-    assert K.dkdv_scan_ints(1, 1, 512, 512, 100, 64, False) == 8 * 512 * 100
-    assert K.dkdv_scan_ints(1, 1, 512, 512, 100, 64, True) == sum(512 - 64 * j for j in range(8)) * 100
-    assert K.dkdv_scan_ints(2, 6, 512, 512, 100, 64, True) <= K.DKDV_SCAN_LIMIT          # the reference's size
-    assert K.dkdv_scan_ints(1, 16, 16384, 16384, 2100, 128, True) > K.DKDV_SCAN_LIMIT    # config 3's shape
+    most = K.SORTED_MAX_POSITIONS
+    assert K.sorted_by_default(512, 512) and K.sorted_by_default(32768, 32768) and K.sorted_by_default(most, most)
+    assert not K.sorted_by_default(most + 1, 64) and not K.sorted_by_default(64, most + 1)
 
 
 def test_tracing_builds_are_separate():

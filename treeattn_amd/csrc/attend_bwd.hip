@@ -7,7 +7,7 @@
 // a candidate row names a key), then 64 / L slots at a time are worked on by L lanes each (L lanes of 8 dimensions
 // hold a row): the key and value rows are read once, in whole lines, the two dot products are finished inside the
 // group, and dq takes the key row that is still in registers.  dk and dv then take one of two routes:
-//  * with a workspace (the Python binding's default while its bound holds): every valid slot's ds and p are written
+//  * with a workspace (the Python binding's default up to 131072 positions): every valid slot's ds and p are written
 //    there, the slots are sorted by key in a stable order (queries ascending, slots ascending) and
 //    bwd_keys_kernel adds each key's contributions from its own consecutive list.  Which entries a lane adds, and
 //    how the lanes' and wavefronts' parts are added, follows from the list alone: dk and dv are bit-reproducible.

@@ -90,8 +90,9 @@ class _SparseAttnFn(torch.autograd.Function):
 
 def sparse_attn(q, k, v, cand, scale, causal=False):
     """cand: (b,H,T,K) int, -1 = unused slot (fastseg.py:173-177).  Differentiable in q, k, v; the gradients
-    of k and v are summed in a fixed order (bit-reproducible).  causal (no counterpart in the reference): every
-    candidate position is at most its query's position, which lets the backward skip work."""
+    of k and v are summed in a fixed order (bit-reproducible) up to 131072 queries and keys, with atomic adds past that
+    (kernels.SORTED_MAX_POSITIONS).  causal (no counterpart in the reference): every candidate position is at most its
+    query's position."""
     _use_fast(q)
     if torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v)):
         return _SparseAttnFn.apply(q, k, v, cand, scale, causal)

@@ -635,19 +635,16 @@ def sparse_attn_fwd(q, k, v, cand, scale):
     return out, lse
 
 
-# Where the default leaves the deterministic dk/dv route for the atomic one, as a count that grows with the square
-# of T (dkdv_scan_ints).  The deterministic route sorts the slots by key, whose time is linear in them, but holds 16
-# bytes per candidate slot while the backward runs; the line keeps that below a few GB at training lengths.
-DKDV_SCAN_LIMIT = 2 ** 31
+# The default route of dk and dv: the fixed order up to this many queries and keys, atomic adds past it.  What grows is
+# the list of the key that every query names: one workgroup adds it.  Milliseconds, fixed order / atomic adds, bfloat16
+# heads of 64, 52 slots a query of which a quarter name a key: (1, 6, 32768) 1.29 / 3.30, (1, 1, 65536) 1.69 / 1.93,
+# (1, 6, 131072) 5.7 / 12.9, (1, 1, 131072) 4.0 / 3.8, (1, 1, 262144) 12.1 / 7.6, (1, 6, 262144) 26.8 / 23.2.
+SORTED_MAX_POSITIONS = 2 ** 17
 
 
-def dkdv_scan_ints(B, H, T, Tk, KC, D, causal):
-    """Candidate entries at or after each block of 4096 / D keys (causal; else all of them), over the blocks: what
-    DKDV_SCAN_LIMIT bounds."""
-    KB = max(1, 4096 // max(D, 1))
-    nblk = (Tk + KB - 1) // KB
-    rows = sum(T - min(j * KB, T) for j in range(nblk)) if causal else nblk * T
-    return B * H * rows * KC
+def sorted_by_default(T, Tk):
+    """Whether sparse_attn_bwd sums dk and dv in the fixed order when it is not told."""
+    return max(T, Tk) <= SORTED_MAX_POSITIONS
 
 
 def _read_rows(t):
@@ -668,10 +665,10 @@ def _grad_rows(t, alloc, dtype):
 
 def sparse_attn_bwd(q, k, v, cand, scale, out, lse, dout, deterministic=None, causal=False):
     """Gradients of sparse_attn_fwd: (dq in q's dtype, dk, dv in k's / v's dtype).  dk and dv are summed in
-    float32: deterministic, in a fixed order (the slots sorted by key, queries then slots ascending) through a
-    per-slot workspace; else with atomic adds whose order depends on scheduling, as in the reference's kernel.
-    deterministic=None (the default) takes the fixed order while dkdv_scan_ints stays within DKDV_SCAN_LIMIT, the
-    atomic adds above it.  causal: every candidate position is at most its query's position."""
+    float32: deterministic, in a fixed order (the slots sorted by key) through a workspace of at most about 1 GiB; else
+    with atomic adds whose order depends on scheduling, as in the reference's kernel.  deterministic=None (the default)
+    takes the fixed order up to SORTED_MAX_POSITIONS queries and keys, the atomic adds past it.  causal: every candidate
+    position is at most its query's position (neither route needs to know)."""
     L.require_gpu(q, k, v, cand, out, lse, dout)
     if not (q.dtype == k.dtype == v.dtype == out.dtype):
         raise TypeError('q, k, v and out must share a dtype')
@@ -684,7 +681,7 @@ def sparse_attn_bwd(q, k, v, cand, scale, out, lse, dout, deterministic=None, ca
     dq = _grad_rows(q, torch.empty, q.dtype)
     ws = None
     if deterministic is None:
-        deterministic = dkdv_scan_ints(b, H, T, Tk, KC, D, causal and T == Tk) <= DKDV_SCAN_LIMIT
+        deterministic = sorted_by_default(T, Tk)
     if deterministic and T > 0 and KC > 0:
         nbytes = L.lib().ta_sparse_attn_bwd_workspace_size(b, H, T, KC)
         ws = torch.empty(max(1, nbytes // 4), device=q.device, dtype=torch.float32)

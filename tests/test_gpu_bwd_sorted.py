@@ -152,6 +152,22 @@ def test_strided_rows_equal_contiguous(dtype, T, H, D, case):
         assert (a.float() - b.float()).abs().max().item() <= tol * max(1.0, b.float().abs().max().item())
 
 
+@pytest.mark.parametrize('T,D,dtype', [(1, 8, torch.float32), (70, 64, torch.float16), (33, 24, torch.bfloat16)])
+def test_contiguous_keys_off_alignment(T, D, dtype):
+    """Contiguous keys and values off a 16-byte boundary, and a single pair with an odd stride of its batch: the bits of
+    the aligned ones."""
+    g = torch.Generator().manual_seed(T)
+    q, k, v, do, out = (torch.randn(1, 1, T, D, generator=g).to(dtype).to(DEV) for _ in range(5))
+    cand = torch.randint(-1, T, (1, 1, T, 9), generator=g).to(DEV)
+    lse = torch.zeros(1, 1, T, device=DEV)
+    want = K.sparse_attn_bwd(q, k, v, cand, 0.1, out, lse, do)
+    off = [torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(1, 1, T, D) for x in (k, v)]
+    odd = [x.as_strided((1, 1, T, D), (3, 5, D, 1)) for x in (k, v)]
+    for kv in (off, odd):
+        assert kv[0].is_contiguous()
+        assert all(torch.equal(a, b) for a, b in zip(K.sparse_attn_bwd(q, *kv, cand, 0.1, out, lse, do), want))
+
+
 def test_atomic_route_adds_whole_lines():
     """The atomic adds go to consecutive dimensions from consecutive lanes: with lanes 32 bytes apart this call took 13.4
     times the sorted route's; consecutive ones take about 3 times (337 against 109 us at 52 slots, a quarter of them

@@ -647,11 +647,13 @@ def sorted_by_default(T, Tk):
     return max(T, Tk) <= SORTED_MAX_POSITIONS
 
 
-def _read_rows(t):
-    """t, or its contiguous copy where the backward's 16-byte reads do not fit its rows."""
+def _read_rows(t, aligned=False):
+    """t, or its contiguous copy where the backward's 16-byte reads do not fit its rows.  A contiguous t off a 16-byte
+    boundary is read one element at a time, unless the rows have to be `aligned` (keys and values): then copied too."""
     es = t.element_size()
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s * es % 16 == 0 for s in t.stride()[:-1])
-    return t if ok else t.contiguous()
+    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s * es % 16 == 0 for s in t.stride()[:-1]):
+        return t
+    return t.clone(memory_format=torch.contiguous_format) if aligned else t.contiguous()
 
 
 def _grad_rows(t, alloc, dtype):
@@ -672,7 +674,8 @@ def sparse_attn_bwd(q, k, v, cand, scale, out, lse, dout, deterministic=None, ca
     L.require_gpu(q, k, v, cand, out, lse, dout)
     if not (q.dtype == k.dtype == v.dtype == out.dtype):
         raise TypeError('q, k, v and out must share a dtype')
-    q, k, v, out, dout = [_read_rows(t) for t in (q, k, v, out, dout.to(q.dtype))]
+    q, out, dout = [_read_rows(t) for t in (q, out, dout.to(q.dtype))]
+    k, v = [_read_rows(t, aligned=True) for t in (k, v)]
     b, H, T, D = q.shape
     Tk = k.shape[2]
     KC = cand.shape[-1]

@@ -210,7 +210,8 @@ int ta_assemble_candidates(const int64_t* tree_pos, const uint8_t* leaf_ok, cons
  * tq[b * tq_sb + n].  Writes n_tree int32 (B,H,N) (the budget split; may be NULL), cm int32 (B,H,N,KC) with KC =
  * (wl + S) * leaf + 1 + max(local, 3) (+ leaf when leaf > 2), entries in ta_assemble_candidates' order (may be NULL),
  * and sums int32 (sum_rows, 5), the columns' sums over sum_rows parts of the rows: kept entries, kept tree entries,
- * kept neighbour entries, leaves used, nL.  wl, S at most 64; leaf a power of two.
+ * kept neighbour entries, leaves used, nL (the first three 0 without cm).  wl, S at most 64; leaf a power of two, at
+ * most 65536 with cm.
  */
 int ta_assemble_leaves(const int32_t* ids, const uint8_t* vld, const int64_t* lhat, const int32_t* nL,
                        const int32_t* nid, const uint8_t* match, const int32_t* tq, int64_t tq_sb, int B, int H,

@@ -47,3 +47,19 @@ def test_list_budgets_and_sums_equal_the_torch_assembly(b, H, N, wl, leaf, Wn, N
     rows = b * H * N
     assert torch.equal(torch.round(means.cpu().double() * rows).long(), want)
     assert torch.equal(means2[3:], means[3:])
+
+
+def test_budgets_of_very_large_leaves():
+    """Budgets and statistics need no list: leaves of more keys than a list's rows can hold."""
+    b, H, N, wl, leaf = 1, 2, 300, 3, 1 << 17
+    g = torch.Generator().manual_seed(1)
+    vld = torch.rand(b, H, N, wl, generator=g) < 0.7
+    ids = torch.where(vld, torch.randint(0, 9, (b, H, N, wl), generator=g), -1)
+    lhat = torch.randint(0, wl + 2, (b, H, N), generator=g)
+    cfg = Config(wmax=wl, leaf=leaf)
+    none, n_tree, means = K.assemble_leaves(ids.int().to(DEV), vld.to(torch.uint8).to(DEV), lhat.to(DEV), cfg, leaf,
+                                            cand=False)
+    want = SEL.budget_split(torch.zeros_like(lhat), lhat, wl)
+    used = (vld & (torch.arange(wl) < want.unsqueeze(-1))).sum()
+    assert none is None and torch.equal(n_tree.cpu().long(), want)
+    assert int(torch.round(means[3].cpu().double() * b * H * N)) == int(used)

@@ -65,6 +65,15 @@ def test_library_rejects_bad_arguments_without_gpu():
     rc = L.ta_assemble_candidates(one, one, one, one, one, 0, 1, 1, 8, 64, 4, 128, 3, one, one, None)
     assert rc == 1
     assert b'at most 320 candidates' in L.ta_last_error()
+    # the list from leaves: leaves of at most 65536 keys (positions are found in float32), 64 leaves of each kind; the
+    # wrapper's callers take the torch assembly where its rule says so
+    from treeattn_amd import kernels as K
+    for wl, leaf, S, local in [(4, 131072, 0, 3), (65, 2, 0, 3), (4, 2, 65, 3), (4, 2, 16, 64)]:
+        assert not K.leaves_supported(wl, leaf, S, local)
+        rc = L.ta_assemble_leaves(one, one, one, one, one, one, one, 0, 1, 1, 8, wl, S, leaf, local, wl, one, one, one,
+                                  1, None)
+        assert rc == 1 and b'at most 65536 for the list' in L.ta_last_error()
+    assert K.leaves_supported(64, 65536, 64, 63) and K.leaves_supported(4, 1 << 20, 0, 3, cand=False)
     # LaneTree workspace: T a power of two in [4, 262144], chunk dividing T, head size 16 / 32 / 64 / 128
     nb = ctypes.c_int64(0)
     assert L.ta_lanetree_workspace_size(1, 6, 131072, 64, 4096, ctypes.byref(nb)) == 0

@@ -283,16 +283,18 @@ extern "C" int ta_assemble_leaves(const int32_t* ids, const uint8_t* vld, const 
   const int lw = local > 3 ? local : 3;
   if (ids == nullptr || vld == nullptr || lhat == nullptr || sums == nullptr || B <= 0 || H <= 0 || N <= 0 || wl < 1 ||
       wl > kWave || S < 0 || S > kWave || (S > 0 && (nid == nullptr || match == nullptr)) || leaf < 2 ||
-      (leaf & (leaf - 1)) || leaf > 65536 || local < 0 || lw >= kWave || wmax < 0 || sum_rows < 1 ||
-      (cm != nullptr && tq == nullptr)) {
+      (leaf & (leaf - 1)) || local < 0 || lw >= kWave || wmax < 0 || sum_rows < 1 ||
+      (cm != nullptr && (tq == nullptr || leaf > 65536))) {
     set_error("ta_assemble_leaves: bad arguments (at most 64 tree leaves and 64 stored ones per row, leaf a power of "
-              "two, local below 64)");
+              "two, at most 65536 for the list, local below 64)");
     return TA_ERR_ARG;
   }
   const int64_t rows = (int64_t)B * H * N;
   const int64_t KC = ((int64_t)wl + S) * leaf + 1 + lw + (leaf > 2 ? leaf : 0);
+  // rows that one row of sums adds up, and the most that one of them adds
   const int64_t per_wave = (rows + (int64_t)sum_rows * kLeafRows - 1) / ((int64_t)sum_rows * kLeafRows);
-  if ((per_wave + kWave) * kLeafRows * KC > 0x7fffffff) {
+  const int64_t most = cm != nullptr ? per_wave * kLeafRows * KC : (per_wave + kWave) * kLeafRows * kWave;
+  if (most > 0x7fffffff) {
     set_error("ta_assemble_leaves: too many rows for the sums");
     return TA_ERR_ARG;
   }

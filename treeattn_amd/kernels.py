@@ -587,9 +587,9 @@ def assemble_candidates(sel, tq, local, leaf, b, H):
     return cm, counts
 
 
-def leaves_supported(wl, leaf, S, local):
-    """Whether assemble_leaves takes these widths."""
-    return 1 <= wl <= 64 and S <= 64 and max(local, 3) < 64
+def leaves_supported(wl, leaf, S, local, cand=True):
+    """Whether assemble_leaves takes these widths; without the list (cand False) a leaf may have any size."""
+    return 1 <= wl <= 64 and S <= 64 and max(local, 3) < 64 and (leaf <= 65536 or not cand)
 
 
 def assemble_leaves(ids, vld, lhat, cfg, leaf, tq=None, nb=None, cand=True):

@@ -223,7 +223,7 @@ def attend(q, k, v, lhat, cfg, scale=None, want_sel=True):
         wl = ids.shape[-1]
         S = cfg.nb_window * cfg.nb_store if nb is not None else 0
         structural = not cfg.neighbors and not grad
-        if K.leaves_supported(wl, leaf, S, cfg.local):
+        if K.leaves_supported(wl, leaf, S, cfg.local, cand=not structural):
             # the candidate list, the budgets and the statistics from the leaves in one launch
             cm, n_tree, m = K.assemble_leaves(ids, vld, lhat, cfg, leaf, tq32, nb, cand=not structural)
             if structural:

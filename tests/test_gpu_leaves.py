@@ -63,3 +63,18 @@ def test_budgets_of_very_large_leaves():
     used = (vld & (torch.arange(wl) < want.unsqueeze(-1))).sum()
     assert none is None and torch.equal(n_tree.cpu().long(), want)
     assert int(torch.round(means[3].cpu().double() * b * H * N)) == int(used)
+
+
+def test_positions_and_budgets_of_other_forms():
+    """int64 or strided positions and a budget that is broadcast: the list of the plain ones."""
+    b, H, N, wl = 2, 3, 50, 5
+    g = torch.Generator().manual_seed(2)
+    vld = torch.rand(b, H, N, wl, generator=g) < 0.7
+    ids = torch.where(vld, torch.randint(0, 9, (b, H, N, wl), generator=g), -1).int().to(DEV)
+    cfg = Config(wmax=wl)
+    t = torch.randint(20, 90, (b, 2 * N), generator=g).to(DEV)
+    one = torch.full((1, 1, 1), 3, device=DEV)
+    args = [ids, vld.to(torch.uint8).to(DEV)]
+    want = K.assemble_leaves(*args, one.expand(b, H, N).contiguous(), cfg, 2, t[:, ::2].int().contiguous())
+    got = K.assemble_leaves(*args, one, cfg, 2, t[:, ::2])
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

@@ -94,6 +94,34 @@ def test_product_refuses_cpu_tensors():
         kernels.gather_dot(q, q, torch.zeros(1, 1, 4, 2, dtype=torch.long), 1.0)
 
 
+def test_assemble_leaves_checks_its_tensors():
+    """Tensors whose memory would be read as something else, or past its end, are refused before any launch."""
+    import torch
+    from treeattn_amd import kernels as K
+    from treeattn_amd.config import Config
+    b, H, N, wl, S = 1, 2, 8, 3, 4
+    ids, vld = torch.zeros(b, H, N, wl, dtype=torch.int32), torch.zeros(b, H, N, wl, dtype=torch.uint8)
+    nb = [torch.zeros(b, H, N, S, dtype=torch.int32), torch.zeros(b, H, N, S, dtype=torch.bool),
+          torch.zeros(b, H, N, dtype=torch.int32)]
+    lhat, tq = torch.ones(b, H, N, dtype=torch.long), torch.arange(N)
+
+    def call(ids=ids, vld=vld, lhat=lhat, tq=tq, nb=nb):
+        K.assemble_leaves(ids, vld, lhat, Config(wmax=wl), 2, tq, nb)
+    with pytest.raises(RuntimeError, match='GPU'):   # all in order but for the device
+        call()
+    wide = torch.zeros(b, H, N, 2 * wl, dtype=torch.int32)
+    for bad in (dict(ids=ids.long()), dict(ids=wide[..., ::2]), dict(ids=ids.transpose(1, 2)), dict(vld=vld.bool()),
+                dict(vld=vld[:, :, :4]), dict(nb=[nb[0].long(), *nb[1:]]), dict(nb=[nb[0], nb[1].to(torch.uint8), nb[2]]),
+                dict(nb=[*nb[:2], nb[2].long()]), dict(nb=[*nb[:2], nb[2][..., :4]])):
+        with pytest.raises(TypeError):
+            call(**bad)
+    for tq in (None, torch.arange(N - 1), torch.zeros(b, H, N)):
+        with pytest.raises(ValueError):
+            call(tq=tq)
+    with pytest.raises(RuntimeError, match='expand'):
+        call(lhat=lhat[..., :4])
+
+
 def test_backward_workspace_is_bounded():
     """The sorted backward's workspace: 16 bytes a slot and the counts of at most 256 chunks of queries, for what is
     sorted at a time -- at most 2^26 slots, or one query's."""

@@ -594,14 +594,23 @@ def leaves_supported(wl, leaf, S, local, cand=True):
 
 def assemble_leaves(ids, vld, lhat, cfg, leaf, tq=None, nb=None, cand=True):
     """The masked candidate list, the leaf budgets and the statistics' means from a selection's leaves in one launch
-    (ta_assemble_leaves): ids int32, vld uint8 (b,H,N,wl) of a descent, lhat (b,H,N) budgets, tq int32 (N,) or (b,N)
+    (ta_assemble_leaves): ids int32, vld uint8 (b,H,N,wl) of a descent, lhat (b,H,N) budgets, tq (N,) or (b,N)
     positions (only needed for the list), nb = (nid int32, match bool, nL int32) of neighbor_pass or None.  Returns
     (cm (b,H,N,KC) int32 or None without `cand`, n_tree (b,H,N) int32, means (5,) float32: kept entries, kept tree
     entries, kept neighbour entries, leaves used, matched leaves, per row)."""
     b, H, N, wl = ids.shape
     nid, match, nL = nb if nb is not None else (None, None, None)
     S = nid.shape[-1] if nid is not None else 0
-    lh = lhat.to(torch.int64).contiguous()
+    for t, dt, shp in ((ids, torch.int32, (b, H, N, wl)), (vld, torch.uint8, (b, H, N, wl)), (nid, torch.int32, (b, H, N, S)),
+                       (match, torch.bool, (b, H, N, S)), (nL, torch.int32, (b, H, N))):
+        if t is not None and (t.dtype != dt or tuple(t.shape) != shp or not t.is_contiguous()):
+            raise TypeError('assemble_leaves: ids int32 and vld uint8 (b,H,N,wl), nid int32 and match bool (b,H,N,S), nL '
+                            'int32 (b,H,N), each contiguous')
+    if tq is not None:
+        tq = tq.to(torch.int32).contiguous()
+    if (tq is None and cand) or (tq is not None and tuple(tq.shape) not in ((N,), (b, N))):
+        raise ValueError('assemble_leaves: positions (N,) or (b,N) for the list')
+    lh = lhat.to(torch.int64).expand(b, H, N).contiguous()
     L.require_gpu(ids, vld, lh, nid, match, nL, tq)
     dev = ids.device
     n_tree = torch.empty(b, H, N, dtype=torch.int32, device=dev)

@@ -267,7 +267,7 @@ int ta_sparse_attn_bwd_strided(const void* q, const void* k, const void* v, cons
                                float* dv, float* ws, int causal, const int64_t* grad_strides, void* stream);
 
 /* Bytes of the deterministic route's workspace of ta_sparse_attn_bwd (per-slot ds and p, the slots sorted by key and
- * the sort's counts); 8-byte aligned. */
+ * the sort's counts); aligned as float32 is. */
 int64_t ta_sparse_attn_bwd_workspace_size(int B, int H, int T, int KC);
 
 /*

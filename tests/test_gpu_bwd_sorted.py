@@ -152,6 +152,28 @@ def test_strided_rows_equal_contiguous(dtype, T, H, D, case):
         assert (a.float() - b.float()).abs().max().item() <= tol * max(1.0, b.float().abs().max().item())
 
 
+def test_workspace_off_alignment():
+    """A workspace aligned to float32 only: the same bits, and nothing past its size is written."""
+    from treeattn_amd import _lib as L
+    B, H, T, KC, D = 1, 2, 90, 7, 16
+    g = torch.Generator().manual_seed(4)
+    q, k, v, o, do = (torch.randn(B, H, T, D, generator=g).to(DEV) for _ in range(5))
+    cand = torch.randint(-1, T, (B, H, T, KC), generator=g, dtype=torch.int32).to(DEV)
+    lse = torch.full((B, H, T), 2.0, device=DEV)
+    words = L.lib().ta_sparse_attn_bwd_workspace_size(B, H, T, KC) // 4
+    got = []
+    for off in (0, 1):
+        buf = torch.full((words + 4,), 7.0, device=DEV)
+        assert buf.data_ptr() % 8 == 0
+        grads = [torch.empty(B, H, T, D, device=DEV) for _ in range(3)]
+        L.call('ta_sparse_attn_bwd', *(L.ptr(x) for x in (q, k, v, o, do)), L.F32,
+               *(s for x in (q, k, v, o, do) for s in L.rows3(x)), L.ptr(cand), L.ptr(lse), B, H, T, T, KC, D, 1.0,
+               *(L.ptr(x) for x in grads), L.ptr(buf[off:]), 0, L.stream())
+        assert bool((buf[off + words:] == 7).all())
+        got.append(grads)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.parametrize('T,D,dtype', [(1, 8, torch.float32), (70, 64, torch.float16), (33, 24, torch.bfloat16)])
 def test_contiguous_keys_off_alignment(T, D, dtype):
     """Contiguous keys and values off a 16-byte boundary, and a single pair with an odd stride of its batch: the bits of

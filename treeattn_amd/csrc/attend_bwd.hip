@@ -622,6 +622,10 @@ static int sparse_attn_bwd_impl(const void* q, const void* k, const void* v, con
     set_error("ta_sparse_attn_bwd: unknown dtype");
     return TA_ERR_ARG;
   }
+  if ((uintptr_t)ws % sizeof(float) != 0) {
+    set_error("ta_sparse_attn_bwd: workspace not aligned to float32");
+    return TA_ERR_ARG;
+  }
   const int es = dtype == TA_F32 ? 4 : 2;
   // key and value rows are read 8 elements at a time
   if (((uintptr_t)k | (uintptr_t)v) % 16 || (ksb * es) % 16 || (ksh * es) % 16 || (kst * es) % 16 ||
@@ -655,9 +659,10 @@ static int sparse_attn_bwd_impl(const void* q, const void* k, const void* v, con
   if (sorted) {
     pl = bwd_plan(B, H, T, KC);
     const int64_t slots = pl.pairs * pl.slots;
-    p.dsp = reinterpret_cast<float2*>(ws);
-    p.ent = reinterpret_cast<uint2*>(ws + 2 * slots);
-    p.cnt = reinterpret_cast<int32_t*>(ws + 4 * slots);
+    float* w = ws + ((uintptr_t)ws % 8 != 0);   // pairs of words; the size has room for the step
+    p.dsp = reinterpret_cast<float2*>(w);
+    p.ent = reinterpret_cast<uint2*>(w + 2 * slots);
+    p.cnt = reinterpret_cast<int32_t*>(w + 4 * slots);
     p.CQ = pl.CQ;
   } else if (ws != nullptr) {   // no slots: every row is zero
     const int64_t n = (int64_t)B * H * Tk * D;
@@ -705,5 +710,5 @@ extern "C" int ta_sparse_attn_bwd_strided(const void* q, const void* k, const vo
 extern "C" int64_t ta_sparse_attn_bwd_workspace_size(int B, int H, int T, int KC) {
   if (B <= 0 || H <= 0 || T <= 0 || KC <= 0) return 0;
   const BwdPlan pl = bwd_plan(B, H, T, KC);
-  return pl.pairs * (4 * pl.slots + pl.words) * (int64_t)sizeof(float);
+  return (pl.pairs * (4 * pl.slots + pl.words) + 1) * (int64_t)sizeof(float);
 }

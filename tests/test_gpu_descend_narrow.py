@@ -12,7 +12,9 @@ DEV = 'cuda'
 
 @pytest.mark.parametrize('T,D,leaf,wmax,Nq,dtype', [
     (1024, 64, 2, 8, 257, torch.float16),     # the fewest queries; a last group of one query
-    (4096, 128, 2, 8, 300, torch.float32),    # candidate rows in three parts
+    (4096, 128, 2, 8, 300, torch.float32),
+    (4096, 128, 2, 8, 515, torch.float32),    # candidate rows in three parts (from 1024 queries on)
+    (1024, 64, 2, 8, 5, torch.float32),       # the fewest queries a pair
     (512, 16, 2, 1, 512, torch.bfloat16),     # a beam of one
     (256, 32, 2, 5, 256, torch.float32),      # every position, an odd beam
     (64, 64, 32, 8, 64, torch.bfloat16),      # one level
@@ -20,7 +22,7 @@ DEV = 'cuda'
 ])
 def test_narrow_descent_matches_oracle(T, D, leaf, wmax, Nq, dtype):
     print('case', T, D, leaf, wmax, Nq, dtype, flush=True)
-    B, H = (3, 2) if Nq < 300 else (1, 2)
+    B, H = (3, 2) if 5 < Nq < 300 else (60, 9) if Nq == 5 else (1, 2)
     g = torch.Generator().manual_seed(T + D + wmax)
     q = torch.randn(B, H, Nq, D, generator=g).to(dtype)
     k = torch.randn(B, H, T, D, generator=g).to(dtype)
@@ -73,3 +75,33 @@ def test_wide_descent_matches_oracle(T, D, leaf, arity, wmax, copies):
     ok = want[1]
     assert torch.equal(vld.bool(), ok)
     assert torch.equal(ids.long()[ok], want[0][ok]) and torch.equal(sct[ok], want[2][ok])
+
+
+def _us(f):
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    best = float('inf')
+    for _ in range(6):
+        a.record()
+        for _ in range(8):
+            f()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1000 / 8)
+    return best
+
+
+def test_few_queries_per_pair_keep_their_wavefronts():
+    """One query of each of 2048 (sequence, head) pairs at D = 128, as a decode step asks: with a 16-lane group per query,
+    15 of a workgroup's 16 idle, this took 1.9 times the wavefronts per query, which a beam of 9 still takes."""
+    T, D, w = 4096, 128, 8
+    shape = K.TreeShape(T, 2, 2)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    k = torch.randn(1, 4, T, D, generator=g, device=DEV)
+    lv = [x.expand(512, 4, -1, -1) for x in K.level_sums(k, shape.blevels)]
+    q = torch.randn(512, 4, 1, D, generator=g, device=DEV)
+    tq = torch.tensor([T - 5], dtype=torch.int32, device=DEV)
+    out = K.tree_descend(q, lv, tq, shape, w)
+    few = _us(lambda: K.tree_descend(q, lv, tq, shape, w, out=out))
+    # a beam of 9 is past the 16-lane groups: the same work by wavefronts, a ninth more of it
+    out9 = K.tree_descend(q, lv, tq, shape, 9)
+    assert few < 1.25 * _us(lambda: K.tree_descend(q, lv, tq, shape, 9, out=out9))

@@ -625,7 +625,14 @@ struct DescendRun {
     // a beam of at most 8 over a binary tree: a 16-lane group per query (wl never exceeds the beam).  From 257
     // queries on: against four wavefronts per query 39 -> 20 us at (1, 6, 512, 64), against one 300 -> 77 us at (2, 6,
     // 4096, 64), 655 -> 148 us at (2, 12, 8192, 64) over leaves of 32; up to 256 both take what a launch takes.
-    if (!ap && arity_log2 == 1 && wmax <= kNarrowW && wl <= kNarrowW && nq_all > 256) {
+    // A workgroup takes 16 queries of one (b,h), and at D = 128 a level's rows come in three round trips: with few
+    // queries per (b,h) groups stand idle and the several wavefronts per query are the faster, and at D = 128 with few
+    // queries in all.  us, (pairs, queries each), wavefronts / groups: D = 64 (512, 1) 20.9 / 18.5, (1024, 1) 24 / 28,
+    // (4096, 1) 60 / 89, (1024, 3) 66 / 29; D = 16 (4096, 3) 62 / 70, (4096, 4) 67 / 70; D = 128 (1024, 1) 22 / 44,
+    // (2048, 4) 58 / 96, (512, 8) 27 / 34, (512, 12) 45 / 38, (1024, 16) 115 / 75, (24, 17) 17.9 / 22.3, (4, 250) 20.0 /
+    // 21.8.
+    const bool filled = D <= 64 ? Nq >= 5 || B * H <= 512 : Nq >= 12 && nq_all >= 1024;
+    if (!ap && arity_log2 == 1 && wmax <= kNarrowW && wl <= kNarrowW && nq_all > 256 && filled) {
       hipLaunchKernelGGL((descend_narrow_kernel<T, D>), dim3((Nq + 15) / 16, B * H), dim3(256), 0, st, (const T*)q, qsb,
                          qsh, qsn, H, Nq, Tgeo, tq, tq_sb, lv, n_levels, wmax, wl, ids, vld, sct, so ? *so : no_store);
       return check_launch("descend_narrow_kernel");

@@ -646,10 +646,11 @@ struct DescendRun {
     } else {
       if (wpq == 16) TA_DESC(16, 1024, false, false);
       else if (wide) TA_DESC(4, 256, false, false);
-      // wide lists cut before they are ranked: 65 candidates 3.94 -> 3.58 ms (4, 16, 16384, 128) and 766 -> 727 us
-      // (3, 12, 8192, 64), 131 candidates 296 -> 262 us.  Up to 40 candidates, or 64 leaves before the last query
-      // (positions usually run to Nq), counting the ranks is the faster: 434 against 486 us at 33 candidates.
-      else if (arity * wmax + arity - 1 > 40 && (Nq >> lv.blevel[0]) > kWave) TA_DESC_S(1, 256, false, false, true);
+      // wide lists cut before they are ranked: 65 candidates 3.94 -> 3.58 ms (4, 16, 16384, 128) and 565 -> 502 us
+      // (2, 8, 8192, 64), 131 candidates 296 -> 262 us.  Up to one candidate a lane, or 64 leaves before the last query
+      // (positions usually run to Nq), counting the ranks is as fast or faster: ranked / cut 434 / 486 us at 33
+      // candidates, 446 / 456 at 41, 329 / 336 at 51 of arity 4, 274 / 282 at 47 of arity 8, 449 / 441 at 63.
+      else if (arity * wmax + arity - 1 > kWave && (Nq >> lv.blevel[0]) > kWave) TA_DESC_S(1, 256, false, false, true);
       else TA_DESC(1, 256, false, false);
     }
 #undef TA_DESC

@@ -100,17 +100,21 @@ __global__ __launch_bounds__(256) void level_pass_kernel(const T* __restrict__ i
 
 // The same pass with each thread holding VEC = 16 / sizeof(T) consecutive dimensions of a row, read with one
 // 16-byte load per row: TPR = D / VEC threads cover a row, so a wavefront's load instruction reads whole row
-// slices of 64 / TPR rows (16 rows apart).  Thread (slice, seg):
-// dimensions [slice VEC, slice VEC + VEC) of a segment of 16 consecutive rows, all requested at once, reduced by
-// adjacent pairs with a carry stack; the workgroup's NSEG = 1024 / TPR segment sums are then combined pairwise in
-// LDS, one tree level per step.  Every node is (left + right) of its two children, so the nodes equal level_pass_kernel's bit for
-// bit whatever the thread layout.  Rows, level rows and the strides must keep 16-byte slices aligned.
-// A short sequence gives a few workgroups only and the serial chain of a segment is the time: 1024 threads with
-// segments of 16 rows cover the chunk that 256 threads with segments of 64 did, so the passes are the same.
-// (1, 6, 1024, 64) float16 over pairs of keys 23.6 -> 13.6 us, (2, 6, 4096, 64) 30.9 -> 20.6, (3, 12, 3001, 64) bfloat16 with
-// leaves of 64 19.4 -> 11.7, (4, 16, 16384, 128) 74 -> 68 us.
-constexpr int kVecThreads = 1024;
-constexpr int kVecSeg = 16;   // rows per segment
+// slices of 64 / TPR rows (SEG rows apart), and each thread keeps 16 rows in flight.  Thread (slice, seg):
+// dimensions [slice VEC, slice VEC + VEC) of a segment of SEG consecutive rows, reduced by adjacent pairs with a carry
+// stack; the workgroup's NSEG = THREADS / TPR segment sums are then combined pairwise in LDS, one tree level per step.
+// Every node is (left + right) of its two children, so the nodes equal level_pass_kernel's bit for bit whatever the
+// thread layout.  Rows, level rows and the strides must keep 16-byte slices aligned.
+// The chunk of a workgroup is the same for both layouts (SEG * NSEG rows).  With few workgroups the serial chain of a
+// segment is the time: 1024 threads with segments of 16 rows; us, 256 / 1024 threads: (1, 6, 1024, 64) float16 over
+// pairs of keys 21.8 / 18.4, (2, 6, 4096, 64) 26.8 / 19.6, (4, 12, 16384, 64) bfloat16 with leaves of 64 38 / 32.5,
+// (4, 16, 16384, 128) 79 / 68.  Once the chip is full of whole chunks memory is, and the shorter combination of 64-row
+// segments wins: (32, 12, 16384, 32) float16 105 / 118, (32, 12, 16384, 128) bfloat16 350 / 370, at D = 64 198 / 205.
+// Where the line lies: at more than one workgroup a CU 256 threads are never the slower, but with whole chunks of 1024
+// or 2048 rows 1024 threads keep ahead up to 1024 workgroups: us, 256 / 1024 threads, bfloat16 D = 64: 700 workgroups 53.5
+// / 43.4, 1300 89 / 97, 768 of which half are short 33 / 41; D = 32 (chunks of 4096) 280 workgroups 24.9 / 27.0; float32
+// D = 128 (chunks of 512) 530 workgroups 30.7 / 33.5.
+constexpr int kVecChunk = 64 * 256;       // THREADS * SEG
 template <typename T>
 struct VecPass {
   static constexpr int VEC = 16 / (int)sizeof(T);
@@ -129,16 +133,17 @@ __device__ __forceinline__ void store_node_vec(const LevelOut& lo, int blevel, i
   }
 }
 
-template <typename T, int D>
-__global__ __launch_bounds__(kVecThreads) void level_vec_kernel(const T* __restrict__ in, int64_t isb, int64_t ish,
-                                                        int64_t isr, int H, int n_rows, int base, int zero_first,
-                                                        LevelOut lo, float* __restrict__ tot, int n_chunks) {
+template <typename T, int D, int THREADS>
+__global__ __launch_bounds__(THREADS) void level_vec_kernel(const T* __restrict__ in, int64_t isb, int64_t ish,
+                                                            int64_t isr, int H, int n_rows, int base, int zero_first,
+                                                            LevelOut lo, float* __restrict__ tot, int n_chunks) {
   constexpr int VEC = VecPass<T>::VEC;
   constexpr int TPR = D / VEC;
-  constexpr int NSEG = kVecThreads / TPR;
+  constexpr int NSEG = THREADS / TPR, SEG = kVecChunk / THREADS;
   constexpr int LOG_NSEG = __builtin_ctz(NSEG);
-  constexpr int LSEG = __builtin_ctz(kVecSeg);
-  static_assert(TPR >= 1 && (1 << LOG_NSEG) == NSEG && (1 << LSEG) == kVecSeg, "layout");
+  constexpr int LSEG = __builtin_ctz(SEG);
+  constexpr int RB = 8;    // rows per load batch; two batches in flight
+  static_assert(TPR >= 1 && (1 << LOG_NSEG) == NSEG && (1 << LSEG) == SEG && SEG % (2 * RB) == 0, "layout");
   __shared__ __align__(16) float seg_sum[NSEG][D];
   const int sl = threadIdx.x % TPR;
   const int seg = threadIdx.x / TPR;
@@ -146,42 +151,54 @@ __global__ __launch_bounds__(kVecThreads) void level_vec_kernel(const T* __restr
   const int chunk = blockIdx.x;
   const int bh = blockIdx.y;
   const int b = bh / H, h = bh % H;
-  const int64_t crow0 = (int64_t)chunk * kVecSeg * NSEG;
-  const int64_t row0 = crow0 + seg * kVecSeg;
+  const int64_t crow0 = (int64_t)chunk * SEG * NSEG;
+  const int64_t row0 = crow0 + seg * SEG;
   const T* src = in + b * isb + h * ish + d0;
   const int64_t last = n_rows - 1;
 
   float carry[LSEG + 1][VEC];
-  uint4 buf[kVecSeg];
+  uint4 buf[2][RB];
 #pragma unroll
-  for (int i = 0; i < kVecSeg; ++i) {
+  for (int i = 0; i < RB; ++i) {
     const int64_t r = row0 + i < last ? row0 + i : last;
-    buf[i] = ldg16(src + r * isr);
+    buf[0][i] = ldg16(src + r * isr);
   }
 #pragma unroll
-  for (int i = 0; i < kVecSeg; ++i) {
-    const int64_t r = row0 + i;
-    if (r < n_rows) {
-      float x[VEC];
-      const T* e = reinterpret_cast<const T*>(&buf[i]);
+  for (int bt = 0; bt < SEG / RB; ++bt) {
+    if (bt + 1 < SEG / RB) {
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) {
-        x[v] = (zero_first && r == 0) ? 0.0f : to_f32(e[v]);
+      for (int i = 0; i < RB; ++i) {
+        const int64_t rr = row0 + (bt + 1) * RB + i;
+        const int64_t r = rr < last ? rr : last;
+        buf[(bt + 1) & 1][i] = ldg16(src + r * isr);
       }
-      int lv = 0;
+    }
 #pragma unroll
-      for (int k = 0; k < LSEG; ++k) {
-        if (((i >> k) & 1) == 0) break;
+    for (int i0 = 0; i0 < RB; ++i0) {
+      const int i = bt * RB + i0;
+      const int64_t r = row0 + i;
+      if (r < n_rows) {
+        float x[VEC];
+        const T* e = reinterpret_cast<const T*>(&buf[bt & 1][i0]);
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) x[v] = __fadd_rn(carry[k][v], x[v]);
-        lv = k + 1;
-        store_node_vec<VEC>(lo, base + lv, b, h, r >> lv, D, d0, x);
+        for (int v = 0; v < VEC; ++v) {
+          x[v] = (zero_first && r == 0) ? 0.0f : to_f32(e[v]);
+        }
+        int lv = 0;
+#pragma unroll
+        for (int k = 0; k < LSEG; ++k) {
+          if (((i >> k) & 1) == 0) break;
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) x[v] = __fadd_rn(carry[k][v], x[v]);
+          lv = k + 1;
+          store_node_vec<VEC>(lo, base + lv, b, h, r >> lv, D, d0, x);
+        }
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) carry[lv][v] = x[v];
       }
-#pragma unroll
-      for (int v = 0; v < VEC; ++v) carry[lv][v] = x[v];
     }
   }
-  if (row0 + kVecSeg - 1 < n_rows) {
+  if (row0 + SEG - 1 < n_rows) {
 #pragma unroll
     for (int v = 0; v < VEC; v += 4)
       *reinterpret_cast<float4*>(&seg_sum[seg][d0 + v]) =
@@ -192,9 +209,9 @@ __global__ __launch_bounds__(kVecThreads) void level_vec_kernel(const T* __restr
   for (int k = 0; k < LOG_NSEG; ++k) {
     __syncthreads();
     const int npairs = NSEG >> (k + 1);
-    for (int e = threadIdx.x; e < npairs * TPR; e += kVecThreads) {
+    for (int e = threadIdx.x; e < npairs * TPR; e += THREADS) {
       const int p = e / TPR, s2 = e % TPR;
-      const int64_t node_rows = (int64_t)kVecSeg << (k + 1);
+      const int64_t node_rows = (int64_t)SEG << (k + 1);
       if (crow0 + (p + 1) * node_rows <= n_rows) {
         float* lft = &seg_sum[(2 * p) << k][s2 * VEC];
         const float* rgt = &seg_sum[(2 * p + 1) << k][s2 * VEC];
@@ -207,9 +224,9 @@ __global__ __launch_bounds__(kVecThreads) void level_vec_kernel(const T* __restr
       }
     }
   }
-  if (tot != nullptr && crow0 + kVecSeg * NSEG <= n_rows) {
+  if (tot != nullptr && crow0 + SEG * NSEG <= n_rows) {
     __syncthreads();
-    for (int e = threadIdx.x; e < D / 4; e += kVecThreads)
+    for (int e = threadIdx.x; e < D / 4; e += THREADS)
       *reinterpret_cast<float4*>(tot + ((int64_t)bh * n_chunks + chunk) * D + 4 * e) =
           *reinterpret_cast<const float4*>(&seg_sum[0][4 * e]);
   }
@@ -517,8 +534,8 @@ int dispatch_dt_d(int dt, int D, A&&... a) {
 
 int chunk_rows(int D) { return 64 * (256 / D); }
 
-// Rows of the pass's input a workgroup reduces: kVecSeg rows per segment, kVecThreads / (threads per row) segments.
-int chunk_rows_vec(int D, int elem) { return kVecSeg * (kVecThreads / (D / (16 / elem))); }
+// Rows of the pass's input a workgroup reduces: its segments' rows, threads / (threads per row) segments.
+int chunk_rows_vec(int D, int elem) { return kVecChunk / (D / (16 / elem)); }
 
 template <typename T, int D>
 struct LevelSumsRun {
@@ -558,16 +575,20 @@ struct LevelSumsRun {
       float* tot = more ? bufs[pass & 1] : nullptr;
       const int tot_chunks = n_rows / CH;
       dim3 grid(n_chunks, B * H);
-      const dim3 threads(vec ? kVecThreads : 256);
+      const bool many = n_rows >= CH &&
+                        (int64_t)n_chunks * B * H > (n_rows % CH == 0 && (CH == 1024 || CH == 2048) ? 1024 : 256);
+      const dim3 threads(vec && !many ? 1024 : 256);
 #define TA_LEVEL_PASS(KER, TT, ZF)                                                                                 \
   hipLaunchKernelGGL(KER, grid, threads, 0, st, (const TT*)src, sb, sh, sr, H, n_rows, base, ZF, lo, tot, tot_chunks)
       if (pass == 0 && logt) {
         TA_LEVEL_PASS((level_pass_kernel<T, D, true>), T, zero_sink);
       } else if (pass == 0) {
-        if (vec) TA_LEVEL_PASS((level_vec_kernel<T, D>), T, zero_sink);
+        if (vec && many) TA_LEVEL_PASS((level_vec_kernel<T, D, 256>), T, zero_sink);
+        else if (vec) TA_LEVEL_PASS((level_vec_kernel<T, D, 1024>), T, zero_sink);
         else TA_LEVEL_PASS((level_pass_kernel<T, D>), T, zero_sink);
       } else {
-        if (vec) TA_LEVEL_PASS((level_vec_kernel<float, D>), float, 0);
+        if (vec && many) TA_LEVEL_PASS((level_vec_kernel<float, D, 256>), float, 0);
+        else if (vec) TA_LEVEL_PASS((level_vec_kernel<float, D, 1024>), float, 0);
         else TA_LEVEL_PASS((level_pass_kernel<float, D>), float, 0);
       }
 #undef TA_LEVEL_PASS

@@ -659,8 +659,10 @@ def sorted_by_default(T, Tk):
 def _read_rows(t, aligned=False):
     """t, or its contiguous copy where the backward's 16-byte reads do not fit its rows.  A contiguous t off a 16-byte
     boundary is read one element at a time, unless the rows have to be `aligned` (keys and values): then copied too."""
-    es = t.element_size()
-    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s * es % 16 == 0 for s in t.stride()[:-1]):
+    if not aligned and t.is_contiguous():
+        return t
+    sb, sh, st, sd = t.stride()
+    if sd == 1 and t.data_ptr() % 16 == 0 and (sb | sh | st) * t.element_size() % 16 == 0:
         return t
     return t.clone(memory_format=torch.contiguous_format) if aligned else t.contiguous()
 
@@ -700,7 +702,7 @@ def sparse_attn_bwd(q, k, v, cand, scale, out, lse, dout, deterministic=None, ca
     alloc = torch.empty if ws is not None else torch.zeros   # written whole, or accumulated into
     dk = _grad_rows(k, alloc, torch.float32)
     dv = _grad_rows(v, alloc, torch.float32)
-    strides = L.i64_array([s for t in (dq, dk, dv) for s in t.stride()[:3]])
+    strides = L.i64_array(dq.stride()[:3] + dk.stride()[:3] + dv.stride()[:3])
     L.call('ta_sparse_attn_bwd_strided', L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(out), L.ptr(dout), L.dtype_code(q),
            *L.rows3(q), *L.rows3(k), *L.rows3(v), *L.rows3(out), *L.rows3(dout), L.ptr(cc), L.ptr(ls), b, H, T, Tk,
            KC, D, float(scale), L.ptr(dq), L.ptr(dk), L.ptr(dv), L.ptr(ws), 1 if (causal and T == Tk) else 0,

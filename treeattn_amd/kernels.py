@@ -601,14 +601,17 @@ def assemble_leaves(ids, vld, lhat, cfg, leaf, tq=None, nb=None, cand=True):
     b, H, N, wl = ids.shape
     nid, match, nL = nb if nb is not None else (None, None, None)
     S = nid.shape[-1] if nid is not None else 0
-    for t, dt, shp in ((ids, torch.int32, (b, H, N, wl)), (vld, torch.uint8, (b, H, N, wl)), (nid, torch.int32, (b, H, N, S)),
-                       (match, torch.bool, (b, H, N, S)), (nL, torch.int32, (b, H, N))):
-        if t is not None and (t.dtype != dt or tuple(t.shape) != shp or not t.is_contiguous()):
-            raise TypeError('assemble_leaves: ids int32 and vld uint8 (b,H,N,wl), nid int32 and match bool (b,H,N,S), nL '
-                            'int32 (b,H,N), each contiguous')
+    rows3 = ids.shape[:3]
+    if not (ids.dtype == torch.int32 and vld.dtype == torch.uint8 and vld.shape == ids.shape and ids.is_contiguous()
+            and vld.is_contiguous() and (nb is None or (
+                nid.dtype == nL.dtype == torch.int32 and match.dtype == torch.bool and nid.shape == match.shape
+                and nid.shape[:3] == nL.shape == rows3 and nid.is_contiguous() and match.is_contiguous()
+                and nL.is_contiguous()))):
+        raise TypeError('assemble_leaves: ids int32 and vld uint8 (b,H,N,wl), nid int32 and match bool (b,H,N,S), nL '
+                        'int32 (b,H,N), each contiguous')
     if tq is not None:
         tq = tq.to(torch.int32).contiguous()
-    if (tq is None and cand) or (tq is not None and tuple(tq.shape) not in ((N,), (b, N))):
+    if (cand if tq is None else tq.shape != (N,) and tq.shape != (b, N)):
         raise ValueError('assemble_leaves: positions (N,) or (b,N) for the list')
     lh = lhat.to(torch.int64).expand(b, H, N).contiguous()
     L.require_gpu(ids, vld, lh, nid, match, nL, tq)

@@ -285,8 +285,8 @@ def test_sparse_attn_bwd_matches_oracle(dtype, D, KC, det):
 
 @pytest.mark.parametrize('D,KC,T', [(64, 52, 300), (16, 9, 70), (128, 80, 200)])
 def test_sparse_attn_bwd_is_bit_reproducible(D, KC, T):
-    """The fixed-order route: dk and dv (and dq) are the same bits on every run, with and without the causal
-    shortcut (causal candidates: every slot at or before its query), and within float32 rounding of the
+    """The fixed-order route: dk and dv (and dq) are the same bits on every run, whether or not the call says that
+    the candidates are causal (every slot at or before its query), and within float32 rounding of the
     atomic route."""
     print('case', D, KC, T, flush=True)
     B, H = 2, 3

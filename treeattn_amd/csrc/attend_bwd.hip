@@ -16,14 +16,15 @@
 //
 // The sort is one stable most-significant-digit pass over chunks of queries (bwd_count_kernel, bwd_scan_kernel,
 // bwd_scatter_kernel) into at most 2048 buckets of 16 (or more) consecutive keys; bwd_keys_kernel lists a bucket's
-// entries key by key in LDS.  The cost is linear in the slots.  Past 2^26 slots, 2^22 queries or 2^21 keys the pairs
-// and queries are sorted, and the keys summed, in parts one after another, which keeps the order.  Scanning all candidate rows once per block of keys
-// instead (one wavefront per block, a serial chain over the queries, quadratic in T) took 6.2 ms of the 7.0 ms
-// forward and backward of a (2, 6, 4096, 64) float16 layer with 52 candidates a row (12 valid); this takes 0.13 ms:
-// count 8, scan 14, scatter 18 and keys 90 us.  What is left in the key kernel is latency (about 8 us per bucket, six
+// entries key by key in LDS.  The cost is linear in the slots but for the buckets' finding of their keys (wider buckets
+// past 32768 keys).  Past 2^26 slots, 2^22 queries or 2^21 keys the pairs and queries are sorted, and the keys summed,
+// in parts one after another, which keeps the order.  Scanning all candidate rows once per block of keys instead (one
+// wavefront per block, a serial chain over the queries, quadratic in T) took 6.2 ms of the 7.0 ms forward and backward
+// of a (2, 6, 4096, 64) float16 layer with 52 candidates a row (12 valid); this takes 0.13 ms:
+// count 9, scan 14, scatter 19 and keys 82 us.  What is left in the key kernel is latency (about 8 us per bucket, six
 // rounds of workgroups) and the bucket of the sink, which every query names: its workgroups are started first and
-// take 85 us.  8 or 32 keys per bucket, 4 or 16 wavefronts, tiles of 1024 entries: 0.19-0.25 against 0.19 ms for the
-// whole backward.  bwd_query_kernel: 45 us (85 with a lane per slot and a second pass over the key rows).
+// take 82 us.  8 or 32 keys per bucket, 4 or 16 wavefronts, tiles of 1024 entries: 0.19-0.25 against 0.19 ms for the
+// whole backward.  bwd_query_kernel: 42 us (85 with a lane per slot and a second pass over the key rows).
 #include "common.hpp"
 
 namespace ta {

@@ -335,8 +335,8 @@ __global__ __launch_bounds__(WPQ == 16 ? 1024 : 256) void descend_kernel(
 // bookkeeping (about 300 instructions per level for 17 scores).  Here a level's candidate rows are all requested at
 // once, every lane of the group gets every score from the canonical dot's butterfly, lane c keeps candidate c (the
 // seventeenth is known to all), the ranks are counted with row rotations, and only the kept ids go through LDS.
-// Same scores, ranks and outputs.  (2, 6, 4096, 64) float16 over pairs of keys: 77 us against 300 us; (8, 6,
-// 512, 64) float32 29 against 100 us.
+// Same scores, ranks and outputs.  (2, 6, 4096, 64) float16 over pairs of keys: 73 us against 286 us (vector instructions
+// busy 95 % of the time); (8, 6, 512, 64) float32 28 against 100 us.
 constexpr int kNarrowW = 8;
 
 template <typename TQ, int D>
@@ -644,7 +644,7 @@ struct DescendRun {
                      ap ? *ap : none, alv ? *alv : lv, so ? *so : no_store, ga ? *ga : no_gate)
 #define TA_DESC(WPQ, NTH, APP, GT) TA_DESC_S(WPQ, NTH, APP, GT, false)
     // a beam of at most 8 over a binary tree: a 16-lane group per query (wl never exceeds the beam).  From 257
-    // queries on: against four wavefronts per query 39 -> 20 us at (1, 6, 512, 64), against one 300 -> 77 us at (2, 6,
+    // queries on: against four wavefronts per query 39 -> 20 us at (1, 6, 512, 64), against one 286 -> 73 us at (2, 6,
     // 4096, 64), 655 -> 148 us at (2, 12, 8192, 64) over leaves of 32; up to 256 both take what a launch takes.
     // A workgroup takes 16 queries of one (b,h), and at D = 128 a level's rows come in three round trips: with few
     // queries per (b,h) groups stand idle and the several wavefronts per query are the faster, and at D = 128 with few
